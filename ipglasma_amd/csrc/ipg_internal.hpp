@@ -34,8 +34,7 @@ inline void ipg_obs_from_device(const double* o, ipg_observables* q) {
 
 // site-parallel helpers: nblk = total blocks over all events of the launch
 void ipg_launch_step0(const EvDesc* d_evs, int nev, int nblk, hipStream_t st);
-// variant 0: register budget for 1 wave per SIMD, 1: for 2, 2: 4 x 64 site
-// tiles along y, 3: the tiles down 64-wide column strips (same results)
+// variant: the order of the blocks, 0 to 3 (k_step; same results)
 void ipg_launch_step(const EvDesc* d_evs, int nev, int nblk, int it, hipStream_t st, int variant = 0);
 // the step for the blocks [block0, block0 + nblocks) of one event only
 void ipg_launch_step_event(const EvDesc* d_evs, int nev, int block0, int nblocks, int it, hipStream_t st,

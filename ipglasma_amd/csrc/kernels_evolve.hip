@@ -38,148 +38,250 @@ __device__ __forceinline__ Nb neighbours(int s, int N) {
     return n;
 }
 
-// Anti-Hermitian 3x3 in compact form: imaginary parts of the diagonal and the
-// upper off-diagonal entries (the lower ones are -conj of them).
-struct AH {
-    double d[3];
-    cd o[3];  // (0,1), (0,2), (1,2)
-};
-// X - X^+
-__device__ __forceinline__ AH ah_of(const M3& X) {
-    AH a;
-    a.d[0] = 2. * X.e[0].i;
-    a.d[1] = 2. * X.e[4].i;
-    a.d[2] = 2. * X.e[8].i;
-    a.o[0] = X.e[1] - cconj(X.e[3]);
-    a.o[1] = X.e[2] - cconj(X.e[6]);
-    a.o[2] = X.e[5] - cconj(X.e[7]);
-    return a;
-}
-// traceless part of an anti-Hermitian matrix
-__device__ __forceinline__ AH ah_tl(AH a) {
-    const double t = (a.d[0] + a.d[1] + a.d[2]) / 3.0;
-    a.d[0] -= t;
-    a.d[1] -= t;
-    a.d[2] -= t;
-    return a;
-}
 // traceless Hermitian part of  E + i c1 A + i c2 B  (E Hermitian, A, B anti-Hermitian)
-__device__ __forceinline__ M3 e_update(const M3& E, double c1, const AH& A, double c2, const AH& B) {
-    M3 h;
-    double dd[3];
+__device__ __forceinline__ H3 e_update(const H3& E, double c1, const AH& A, double c2, const AH& B) {
+    H3 h;
 #pragma unroll
-    for (int k = 0; k < 3; k++) dd[k] = E.e[4 * k].r - c1 * A.d[k] - c2 * B.d[k];
-    const double t = (dd[0] + dd[1] + dd[2]) / 3.0;
-    h.e[0] = cd{dd[0] - t, 0.};
-    h.e[4] = cd{dd[1] - t, 0.};
-    h.e[8] = cd{dd[2] - t, 0.};
-    const int up[3] = {1, 2, 5}, lo[3] = {3, 6, 7};
+    for (int k = 0; k < 3; k++) h.d[k] = E.d[k] - c1 * A.d[k] - c2 * B.d[k];
+    const double t = (h.d[0] + h.d[1] + h.d[2]) / 3.0;
 #pragma unroll
-    for (int q = 0; q < 3; q++) {
-        cd v = E.e[up[q]] + cd{-c1 * A.o[q].i - c2 * B.o[q].i, c1 * A.o[q].r + c2 * B.o[q].r};
-        h.e[up[q]] = v;
-        h.e[lo[q]] = cconj(v);
+    for (int k = 0; k < 3; k++) {
+        h.d[k] -= t;
+        h.o[k] = E.o[k] + cd{-c1 * A.o[k].i - c2 * B.o[k].i, c1 * A.o[k].r + c2 * B.o[k].r};
     }
     return h;
 }
 
-// (1 + X + X^2/2) with X = i c E  (the n=2 loop of Evolution.cpp:54-68)
-__device__ __forceinline__ M3 taylor2(double c, const M3& E) {
-    M3 X = mul_i(c, E);
-    M3 t = m_one() + 0.5 * X;
-    return m_one() + X * t;
+// What the roles of a site hand each other through LDS: nine doubles a
+// matrix, [value][lane] so that a wavefront's accesses are conflict free.
+constexpr int kRoleSites = 64;  // sites of a block: one wavefront per role
+template <typename X>
+__device__ __forceinline__ void x_put(double (*b)[kRoleSites], int lane, const X& a) {
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        b[k][lane] = a.d[k];
+        b[3 + 2 * k][lane] = a.o[k].r;
+        b[4 + 2 * k][lane] = a.o[k].i;
+    }
+}
+template <typename X>
+__device__ __forceinline__ X x_get(const double (*b)[kRoleSites], int lane) {
+    X a;
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        a.d[k] = b[k][lane];
+        a.o[k] = cd{b[3 + 2 * k][lane], b[4 + 2 * k][lane]};
+    }
+    return a;
 }
 
-#define IPG_PHASE() __builtin_amdgcn_sched_barrier(0)
+// One step.  A block takes 64 consecutive sites with four wavefronts, each in
+// a role of its own (about 460 FP64 multiply-adds a lane each):
+//   0  phi~_x, phi~_y and the commutators [phi~_i, phi] of evolveE; pi, phi
+//   1  the plaquette U_{1,-2}; E1 and U_x
+//   2  the plaquette U_{2,-1}; E2 and U_y
+//   3  the plaquette U_12 (U_21 is its conjugate: the two E updates take its
+//      anti-Hermitian part with opposite signs) and the x - x^ term of pi
+// The stencil is staged in LDS: the sites of the rows i, i+1 and i-1 are
+// loaded once (117 planes, all loads of a wavefront in flight together and
+// before anything is computed) and the roles read their matrices from there;
+// loaded by each role itself the stencil is 333 planes.
+//   planes  0 U_x(i), 18 U_y(i), 36 U_y(i+1), 54 U_x(i-1), 72 U_y(i-1),
+//          90 phi(i), 99 phi(i+1), 108 phi(i-1)
+// A y neighbour is the next lane's value; the two sites past the ends of the
+// block are in `ends` (108 values).
+constexpr int kSUxI = 0, kSUyI = 18, kSUyP = 36, kSUxM = 54, kSUyM = 72, kSPhI = 90, kSPhP = 99, kSPhM = 108;
+constexpr int kStagePlanes = 117;
+constexpr int kEUxI = 0, kEUxM = 18, kEPhP = 36;                  // right end: U_x(i), U_x(i-1), phi(i)
+constexpr int kELUxI = 45, kELUyI = 63, kELUyP = 81, kELPh = 99;  // left end: U_x(i), U_y(i), U_y(i+1), phi(i)
+constexpr int kStageEnds = 108;
+typedef double StageRow[kRoleSites];
 
-// OCC: waves per SIMD the register budget is sized for (1: no spill, 2:
-// half the registers).  TILED: a block takes a tile of 4 rows x 64 sites (one
-// wavefront per row, coalesced along y as in the row-major mapping) instead
-// of 256 consecutive sites, so that the x-neighbour rows a block reads are
-// mostly its own (events with N a multiple of 64; others keep the row-major
-// mapping); tiles follow each other along y (TILED 1) or down a 64-wide
-// column strip along x (TILED 2), so that the blocks in flight on an XCD
-// share their halo rows.  The autotuner picks the build; the results are
-// identical.
-template <int OCC, int TILED = 0>
-__global__ __launch_bounds__(IPG_BLOCK, OCC) void k_step(const EvDesc* __restrict__ evs, int nev, int it, int b0) {
+template <int NP>
+__device__ __forceinline__ void stage_planes(StageRow* to, const double* f, size_t S, size_t s, int lane) {
+    double v[NP];
+    const unsigned ob = lane_offset<false>(s);
+#pragma unroll
+    for (int k = 0; k < NP; k++) v[k] = gld(f, k * S, ob);
+#pragma unroll
+    for (int k = 0; k < NP; k++) to[k][lane] = v[k];
+}
+// matrix at lane q of the stage
+__device__ __forceinline__ M3 st_m(const StageRow* f, int q) {
+    M3 m;
+#pragma unroll
+    for (int k = 0; k < 9; k++) m.e[k] = cd{f[2 * k][q], f[2 * k + 1][q]};
+    return m;
+}
+__device__ __forceinline__ H3 st_h(const StageRow* f, int q) {
+    H3 h;
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        h.d[k] = f[k][q];
+        h.o[k] = cd{f[3 + 2 * k][q], f[4 + 2 * k][q]};
+    }
+    return h;
+}
+// the same with the value past the block's end taken from `ends`
+__device__ __forceinline__ M3 st_me(const StageRow* f, int q, const double* end, bool past) {
+    const double* b = past ? end : &f[0][q];
+    const int w = past ? 1 : kRoleSites;
+    M3 m;
+#pragma unroll
+    for (int k = 0; k < 9; k++) m.e[k] = cd{b[(2 * k) * w], b[(2 * k + 1) * w]};
+    return m;
+}
+__device__ __forceinline__ H3 st_he(const StageRow* f, int q, const double* end, bool past) {
+    const double* b = past ? end : &f[0][q];
+    const int w = past ? 1 : kRoleSites;
+    H3 h;
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        h.d[k] = b[k * w];
+        h.o[k] = cd{b[(3 + 2 * k) * w], b[(4 + 2 * k) * w]};
+    }
+    return h;
+}
+
+// One thread per site with everything in registers took 382 of them, one
+// wavefront per SIMD, whose chain of loads and products set the pace: 17 us a
+// launch at N = 128 (64 blocks of 256 sites left 192 CUs idle), 26 us at
+// N = 256, 83 us at N = 512; in roles 8.1, 20.4 and 65.6 us (302 MB of fields
+// read and written at N = 512: 4.6 TB/s, a large device copy runs at 4.9).
+// Also measured: each role loading its own matrices (168 registers, three
+// waves per SIMD) 8.7, 20.7, 71 us; at 128 registers it spills (131 us);
+// only row i staged 8.0, 21.6, 68 us; blocks that stay and fetch the next
+// tile while they store the last 12, 28, 97 us (256 registers and spills).
+// order (the tuner's choice; the same results): bit 0: blocks follow each
+// other down 64-wide column strips (N a multiple of 64) instead of along the
+// rows; bit 1: in the hardware's block order instead of a run of rows per XCD.
+__global__ __launch_bounds__(4 * kRoleSites, 2) void k_step(const EvDesc* __restrict__ evs, int nev, int it, int b0,
+                                                            int order) {
     // b0: first block of a launch that covers one event's blocks only (a
     // multiple of 8, so the XCD of a block is unchanged)
+    __shared__ StageRow stage[kStagePlanes];
+    __shared__ double ends[kStageEnds];
+    __shared__ double xch[4][9][kRoleSites];
+    constexpr int B4 = IPG_BLOCK / kRoleSites;
     const int bg = (int)blockIdx.x + b0;
-    const int e = find_event(evs, nev, bg);
+    const int e = find_event(evs, nev, bg / B4);
     const EvDesc& ev = evs[e];
     if (!ev.active || it > ev.itmax) return;
-    const int lb = xcd_remap(bg - ev.block0, ev.nblocks);
-    long long s;
-    if (TILED && (ev.N & 63) == 0) {
-        static_assert(IPG_BLOCK == 256, "4 x 64 tiles");
-        const int tpr = ev.N >> 6;  // tiles along y
-        const int tpc = ev.N >> 2;  // tiles along x
-        if (lb >= tpc * tpr) return;
-        const int ti = TILED == 1 ? lb / tpr : lb % tpc;
-        const int tj = TILED == 1 ? lb - ti * tpr : lb / tpc;
-        s = (long long)(ti * 4 + (int)(threadIdx.x >> 6)) * ev.N + tj * 64 + (int)(threadIdx.x & 63);
-    } else {
-        s = (long long)lb * IPG_BLOCK + threadIdx.x;
-        if (s >= ev.S) return;
+    int lb = bg - B4 * ev.block0;
+    if (!(order & 2)) lb = xcd_remap(lb, B4 * ev.nblocks);
+    const int lane = (int)(threadIdx.x & 63);
+    const int role = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int N = ev.N;
+    if ((order & 1) && (N & 63) == 0) {
+        const int tj = lb / N;
+        lb = (lb - tj * N) * (N >> 6) + tj;
     }
+    // N is a multiple of 16, S of 256: a block is full or past the end
+    if ((long long)lb * kRoleSites >= ev.S) return;
+    const size_t s = (size_t)lb * kRoleSites + lane;
     const size_t S = ev.S;
     const int p = (it - 1) & 1;
     const double tau = it * ev.dtau;
     const bool half = it == ev.itmax;
     const double dt = half ? ev.dtau / 2. : ev.dtau;
-    const Nb n = neighbours((int)s, ev.N);
+    const int i = (int)s / N, j = (int)s - i * N;
+    const size_t pX = (size_t)min(i + 1, N - 1) * N + j, mX = (size_t)max(i - 1, 0) * N + j;
     const double* __restrict__ Ux = ev.U[p][0];
     const double* __restrict__ Uy = ev.U[p][1];
     const double* __restrict__ phi = ev.phi[p];
-
-    // phase 1: pi (evolvePi) and the commutators [phi~_i, phi] of evolveE
-    M3 ux = ldm(Ux, S, s), uy;
-    AH c1, c2;
-    M3 pin;
-    {
-        const M3 ph = ldh(phi, S, s);
-        M3 t = ux * mul_bd(ldh(phi, S, n.pX), ux);  // phi~_x
-        c1 = ah_of(t * ph);
-        M3 br = t;
-        {
-            M3 u = ldm(Ux, S, n.mX);
-            br = br + mul_ad(u, ldh(phi, S, n.mX)) * u;
+    // lane of the y neighbours (clamped), past the block's end or not
+    const bool up = j < N - 1, dn = j > 0;
+    const int qp = up ? min(lane + 1, 63) : lane, qm = dn ? max(lane - 1, 0) : lane;
+    const bool ep = up && lane == 63, em = dn && lane == 0;
+    H3 own;
+    if (role == 0) {
+        own = ldh3(ev.pi, S, s);
+        stage_planes<18>(stage + kSUxI, Ux, S, s, lane);
+        stage_planes<9>(stage + kSPhI, phi, S, s, lane);
+        // right end: the sites of the y neighbour of lane 63 (that lane's own where clamped)
+        const int i63 = __builtin_amdgcn_readlane(i, 63), j63 = min(__builtin_amdgcn_readlane(j, 63) + 1, N - 1);
+        const size_t r = (size_t)i63 * N + j63, rm = (size_t)max(i63 - 1, 0) * N + j63;
+        if (lane < 45) {
+            const double* f = lane < 18 ? Ux + lane * S + r : lane < 36 ? Ux + (lane - 18) * S + rm : phi + (lane - 36) * S + r;
+            ends[lane] = *f;
         }
-        uy = ldm(Uy, S, s);
-        t = uy * mul_bd(ldh(phi, S, n.pY), uy);  // phi~_y
-        c2 = ah_of(t * ph);
-        br = br + t;
-        {
-            M3 u = ldm(Uy, S, n.mY);
-            br = br + mul_ad(u, ldh(phi, S, n.mY)) * u;
+    } else if (role == 1) {
+        own = ldh3(ev.E1, S, s);
+        stage_planes<18>(stage + kSUyI, Uy, S, s, lane);
+        stage_planes<9>(stage + kSPhP, phi, S, pX, lane);
+        const int i0 = __builtin_amdgcn_readfirstlane(i), jm = max(__builtin_amdgcn_readfirstlane(j) - 1, 0);
+        const size_t l = (size_t)i0 * N + jm, lp = (size_t)min(i0 + 1, N - 1) * N + jm;
+        if (lane < 63) {
+            const double* f = lane < 18   ? Ux + lane * S + l
+                              : lane < 36 ? Uy + (lane - 18) * S + l
+                              : lane < 54 ? Uy + (lane - 36) * S + lp
+                                          : phi + (lane - 54) * S + l;
+            ends[kELUxI + lane] = *f;
         }
-        br = br - 4. * ph;
-        pin = herm_part(ldh(ev.pi, S, s) + (dt / tau) * br);
-        sth(ev.pio, S, s, pin);
-        if (!half) sth(ev.phi[p ^ 1], S, s, ph + ((tau + dt / 2.) * dt) * pin);  // evolvePhi
+    } else if (role == 2) {
+        own = ldh3(ev.E2, S, s);
+        stage_planes<18>(stage + kSUyP, Uy, S, pX, lane);
+        stage_planes<9>(stage + kSPhM, phi, S, mX, lane);
+    } else {
+        stage_planes<18>(stage + kSUxM, Ux, S, mX, lane);
+        stage_planes<18>(stage + kSUyM, Uy, S, mX, lane);
     }
-    IPG_PHASE();
+    __syncthreads();
     const double a1 = tau * dt / (2. * ev.g * ev.g);
     const double a2 = dt / tau;
     const double cu = ev.g * ev.g * dt / (tau + dt / 2.);
-    // phase 2: E1 from the plaquettes U_12 and U_{1,-2} (evolveE), then U_x
-    M3 U12 = (ux * ldm(Uy, S, n.pX)) * mul_bd(dag(ldm(Ux, S, n.pY)), uy);
-    {
-        M3 P = mul_bd(ux, ldm(Uy, S, n.pXmY)) * mul_ad(ldm(Ux, S, n.mY), ldm(Uy, S, n.mY));
-        const AH t1 = ah_tl(ah_of(U12 + P));
-        const M3 e1n = e_update(ldh(ev.E1, S, s), a1, t1, a2, c1);
-        sth(ev.E1o, S, s, e1n);
-        if (!half) stm(ev.U[p ^ 1][0], S, s, taylor2(cu, e1n) * ux);  // evolveU
-    }
-    IPG_PHASE();
-    // phase 3: E2 from U_21 = U_12^+ and U_{2,-1}, then U_y
-    {
-        M3 P = mul_bd(uy, ldm(Ux, S, n.mXpY)) * mul_ad(ldm(Uy, S, n.mX), ldm(Ux, S, n.mX));
-        const AH t1 = ah_tl(ah_of(dag(U12) + P));
-        const M3 e2n = e_update(ldh(ev.E2, S, s), a1, t1, a2, c2);
-        sth(ev.E2o, S, s, e2n);
-        if (!half) stm(ev.U[p ^ 1][1], S, s, taylor2(cu, e2n) * uy);
+    if (role == 0) {
+        const H3 ph = st_h(stage + kSPhI, lane);
+        H3 br;
+        {
+            const M3 u = st_m(stage + kSUxI, lane);
+            br = herm_mul(u, mul_hd(st_h(stage + kSPhP, lane), u));  // phi~_x
+            x_put(xch[0], lane, commutator(br, ph));
+        }
+        {
+            const M3 u = st_m(stage + kSUyI, lane);
+            const H3 t = herm_mul(u, mul_hd(st_he(stage + kSPhI, qp, ends + kEPhP, ep), u));  // phi~_y
+            x_put(xch[1], lane, commutator(t, ph));
+            br = br + t;
+        }
+        {
+            const M3 u = st_me(stage + kSUyI, qm, ends + kELUyI, em);
+            br = br + herm_mul_ad(u, mul_h(st_he(stage + kSPhI, qm, ends + kELPh, em), u));
+        }
+        __syncthreads();
+        br = (br + x_get<H3>(xch[3], lane)) + (-4.) * ph;
+        const H3 pin = own + a2 * br;
+        sth3(ev.pio, S, s, pin);
+        if (!half) sth3(ev.phi[p ^ 1], S, s, ph + ((tau + dt / 2.) * dt) * pin);  // evolvePhi
+    } else if (role == 3) {
+        {
+            const M3 u = st_m(stage + kSUxM, lane);
+            x_put(xch[3], lane, herm_mul_ad(u, mul_h(st_h(stage + kSPhM, lane), u)));
+        }
+        {
+            const M3 A = st_m(stage + kSUxI, lane) * st_m(stage + kSUyP, lane);
+            x_put(xch[2], lane,
+                  ah_mul(A, dag(st_m(stage + kSUyI, lane) * st_me(stage + kSUxI, qp, ends + kEUxI, ep))));
+        }
+        __syncthreads();
+    } else {
+        M3 u;
+        AH A;
+        if (role == 1) {
+            u = st_m(stage + kSUxI, lane);
+            const M3 l = mul_bd(u, st_me(stage + kSUyP, qm, ends + kELUyP, em));
+            A = ah_mul(l, mul_ad(st_me(stage + kSUxI, qm, ends + kELUxI, em), st_me(stage + kSUyI, qm, ends + kELUyI, em)));
+        } else {
+            u = st_m(stage + kSUyI, lane);
+            const M3 l = mul_bd(u, st_me(stage + kSUxM, qp, ends + kEUxM, ep));
+            A = ah_mul(l, mul_ad(st_m(stage + kSUyM, lane), st_m(stage + kSUxM, lane)));
+        }
+        __syncthreads();
+        const AH u12 = x_get<AH>(xch[2], lane);
+        A = ah_tl(role == 1 ? A + u12 : A - u12);
+        const H3 e1 = e_update(own, a1, A, a2, x_get<AH>(xch[role - 1], lane));
+        sth3(role == 1 ? ev.E1o : ev.E2o, S, s, e1);
+        if (!half) stm(ev.U[p ^ 1][role - 1], S, s, taylor2(cu, e1) * u);  // evolveU
     }
 }
 
@@ -196,8 +298,8 @@ __global__ __launch_bounds__(IPG_BLOCK) void k_step0(const EvDesc* __restrict__ 
     M3 ph = ldh(ev.phi[0], S, s) + ((tau + dt / 2.) * dt) * ldh(ev.pi, S, s);
     sth(ev.phi[0], S, s, ph);
     const double cu = ev.g * ev.g * dt / (tau + dt / 2.);
-    stm(ev.U[0][0], S, s, taylor2(cu, ldh(ev.E1, S, s)) * ldm(ev.U[0][0], S, s));
-    stm(ev.U[0][1], S, s, taylor2(cu, ldh(ev.E2, S, s)) * ldm(ev.U[0][1], S, s));
+    stm(ev.U[0][0], S, s, taylor2(cu, ldh3(ev.E1, S, s)) * ldm(ev.U[0][0], S, s));
+    stm(ev.U[0][1], S, s, taylor2(cu, ldh3(ev.E2, S, s)) * ldm(ev.U[0][1], S, s));
 }
 
 // ---- reductions ---------------------------------------------------------------
@@ -602,24 +704,14 @@ __global__ __launch_bounds__(IPG_BLOCK) void k_finish(const EvDesc* __restrict__
 void ipg_launch_step0(const EvDesc* d_evs, int nev, int nblk, hipStream_t st) {
     hipLaunchKernelGGL(k_step0, dim3(nblk), dim3(IPG_BLOCK), 0, st, d_evs, nev);
 }
-// variant 0: k_step<1>, 1: k_step<2>, 2: k_step<1> on 4 x 64 tiles along y,
-// 3: k_step<1> on 4 x 64 tiles down column strips (k_step<2> with opaque
-// lane offsets spills 284 B per lane instead of 508, and still takes 158 us
-// against 83 at N = 512)
 void ipg_launch_step(const EvDesc* d_evs, int nev, int nblk, int it, hipStream_t st, int variant) {
     ipg_launch_step_event(d_evs, nev, 0, nblk, it, st, variant);
 }
+// block0, nblocks: in blocks of IPG_BLOCK sites, as everywhere else
 void ipg_launch_step_event(const EvDesc* d_evs, int nev, int block0, int nblocks, int it, hipStream_t st,
                            int variant) {
-    if (variant == 1)
-        hipLaunchKernelGGL(k_step<2>, dim3(nblocks), dim3(IPG_BLOCK), 0, st, d_evs, nev, it, block0);
-    else if (variant == 2)
-        hipLaunchKernelGGL((k_step<1, 1>), dim3(nblocks), dim3(IPG_BLOCK), 0, st, d_evs, nev, it, block0);
-    else if (variant == 3)
-        hipLaunchKernelGGL((k_step<1, 2>), dim3(nblocks), dim3(IPG_BLOCK), 0, st, d_evs, nev, it, block0);
-
-    else
-        hipLaunchKernelGGL(k_step<1>, dim3(nblocks), dim3(IPG_BLOCK), 0, st, d_evs, nev, it, block0);
+    constexpr int B4 = IPG_BLOCK / kRoleSites;
+    hipLaunchKernelGGL(k_step, dim3(B4 * nblocks), dim3(4 * kRoleSites), 0, st, d_evs, nev, it, B4 * block0, variant);
 }
 void ipg_launch_tmunu(const EvDesc* d_evs, int nev, int nblk, int it, hipStream_t st) {
     hipLaunchKernelGGL(k_tmunu_a, dim3(nblk), dim3(IPG_BLOCK), 0, st, d_evs, nev, it);

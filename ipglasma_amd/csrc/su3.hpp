@@ -242,6 +242,211 @@ __device__ __forceinline__ void sth(double* f, size_t S, size_t s0, const M3& m)
     gst(f, 7 * S, s, m.e[5].r);
     gst(f, 8 * S, s, m.e[5].i);
 }
+// ---- Hermitian and anti-Hermitian matrices in compact form --------------------
+// H3: real diagonal and the entries (0,1), (0,2), (1,2) of a Hermitian matrix.
+// Products with it skip the diagonal's zero imaginary parts and the entries
+// that symmetry gives (90 instead of 108 multiply-adds for H M, 54 for a
+// product known to be Hermitian, 48 for a commutator).
+struct H3 {
+    double d[3];
+    cd o[3];
+};
+template <bool Opaque = false>
+__device__ __forceinline__ H3 ldh3(const double* f, size_t S, size_t s0) {
+    const unsigned s = lane_offset<Opaque>(s0);
+    H3 h;
+    h.d[0] = gld(f, 0, s);
+    h.d[1] = gld(f, S, s);
+    h.d[2] = gld(f, 2 * S, s);
+    h.o[0] = cd{gld(f, 3 * S, s), gld(f, 4 * S, s)};
+    h.o[1] = cd{gld(f, 5 * S, s), gld(f, 6 * S, s)};
+    h.o[2] = cd{gld(f, 7 * S, s), gld(f, 8 * S, s)};
+    return h;
+}
+template <bool Opaque = false>
+__device__ __forceinline__ void sth3(double* f, size_t S, size_t s0, const H3& h) {
+    const unsigned s = lane_offset<Opaque>(s0);
+    gst(f, 0, s, h.d[0]);
+    gst(f, S, s, h.d[1]);
+    gst(f, 2 * S, s, h.d[2]);
+    gst(f, 3 * S, s, h.o[0].r);
+    gst(f, 4 * S, s, h.o[0].i);
+    gst(f, 5 * S, s, h.o[1].r);
+    gst(f, 6 * S, s, h.o[1].i);
+    gst(f, 7 * S, s, h.o[2].r);
+    gst(f, 8 * S, s, h.o[2].i);
+}
+IPG_HD H3 operator+(const H3& a, const H3& b) {
+    H3 c;
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        c.d[k] = a.d[k] + b.d[k];
+        c.o[k] = a.o[k] + b.o[k];
+    }
+    return c;
+}
+IPG_HD H3 operator*(double s, const H3& a) {
+    H3 c;
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        c.d[k] = s * a.d[k];
+        c.o[k] = s * a.o[k];
+    }
+    return c;
+}
+// entry (i, j) of a Hermitian matrix off the diagonal
+IPG_HD cd h_off(const H3& h, int i, int j) {
+    const int k = i + j - 1;  // (0,1) 0, (0,2) 1, (1,2) 2
+    return i < j ? h.o[k] : cconj(h.o[k]);
+}
+// H U^+
+IPG_HD M3 mul_hd(const H3& h, const M3& u) {
+    M3 c;
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+#pragma unroll
+        for (int j = 0; j < 3; j++) {
+            const int k = (i + 1) % 3, l = (i + 2) % 3;
+            c.e[3 * i + j] =
+                (cconj(u.e[3 * j + i]) * h.d[i] + mulc(h_off(h, i, k), u.e[3 * j + k])) + mulc(h_off(h, i, l), u.e[3 * j + l]);
+        }
+    return c;
+}
+// H U
+IPG_HD M3 mul_h(const H3& h, const M3& u) {
+    M3 c;
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+#pragma unroll
+        for (int j = 0; j < 3; j++) {
+            const int k = (i + 1) % 3, l = (i + 2) % 3;
+            c.e[3 * i + j] = (u.e[3 * i + j] * h.d[i] + h_off(h, i, k) * u.e[3 * k + j]) + h_off(h, i, l) * u.e[3 * l + j];
+        }
+    return c;
+}
+// the product A B where it is Hermitian
+IPG_HD H3 herm_mul(const M3& a, const M3& b) {
+    H3 h;
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+        double t = 0.;
+#pragma unroll
+        for (int k = 0; k < 3; k++) t += a.e[3 * i + k].r * b.e[3 * k + i].r - a.e[3 * i + k].i * b.e[3 * k + i].i;
+        h.d[i] = t;
+    }
+#pragma unroll
+    for (int q = 0; q < 3; q++) {
+        const int i = q == 2 ? 1 : 0, j = q == 0 ? 1 : 2;
+        h.o[q] = a.e[3 * i] * b.e[j] + a.e[3 * i + 1] * b.e[3 + j] + a.e[3 * i + 2] * b.e[6 + j];
+    }
+    return h;
+}
+// A^+ B where it is Hermitian
+IPG_HD H3 herm_mul_ad(const M3& a, const M3& b) {
+    H3 h;
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+        double t = 0.;
+#pragma unroll
+        for (int k = 0; k < 3; k++) t += a.e[3 * k + i].r * b.e[3 * k + i].r + a.e[3 * k + i].i * b.e[3 * k + i].i;
+        h.d[i] = t;
+    }
+#pragma unroll
+    for (int q = 0; q < 3; q++) {
+        const int i = q == 2 ? 1 : 0, j = q == 0 ? 1 : 2;
+        h.o[q] = cmul(a.e[i], b.e[j]) + cmul(a.e[3 + i], b.e[3 + j]) + cmul(a.e[6 + i], b.e[6 + j]);
+    }
+    return h;
+}
+// Anti-Hermitian 3x3: imaginary parts of the diagonal and the entries (0,1),
+// (0,2), (1,2) (the lower ones are -conj of them)
+struct AH {
+    double d[3];
+    cd o[3];
+};
+// A B - (A B)^+
+IPG_HD AH ah_mul(const M3& a, const M3& b) {
+    AH h;
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+        double t = 0.;
+#pragma unroll
+        for (int k = 0; k < 3; k++) t += a.e[3 * i + k].r * b.e[3 * k + i].i + a.e[3 * i + k].i * b.e[3 * k + i].r;
+        h.d[i] = 2. * t;
+    }
+#pragma unroll
+    for (int q = 0; q < 3; q++) {
+        const int i = q == 2 ? 1 : 0, j = q == 0 ? 1 : 2;
+        const cd up = a.e[3 * i] * b.e[j] + a.e[3 * i + 1] * b.e[3 + j] + a.e[3 * i + 2] * b.e[6 + j];
+        const cd lo = a.e[3 * j] * b.e[i] + a.e[3 * j + 1] * b.e[3 + i] + a.e[3 * j + 2] * b.e[6 + i];
+        h.o[q] = up - cconj(lo);
+    }
+    return h;
+}
+// t p - p t = t p - (t p)^+ of two Hermitian matrices
+IPG_HD AH commutator(const H3& t, const H3& p) {
+    AH h;
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+        const int k = (i + 1) % 3, l = (i + 2) % 3;
+        const cd tk = h_off(t, i, k), pk = h_off(p, i, k), tl = h_off(t, i, l), pl = h_off(p, i, l);
+        h.d[i] = 2. * ((tk.i * pk.r - tk.r * pk.i) + (tl.i * pl.r - tl.r * pl.i));
+    }
+#pragma unroll
+    for (int q = 0; q < 3; q++) {
+        const int i = q == 2 ? 1 : 0, j = q == 0 ? 1 : 2, m = 3 - i - j;
+        h.o[q] = (p.o[q] * (t.d[i] - t.d[j]) + t.o[q] * (p.d[j] - p.d[i])) +
+                 (h_off(t, i, m) * h_off(p, m, j) - h_off(p, i, m) * h_off(t, m, j));
+    }
+    return h;
+}
+// the traceless part
+IPG_HD AH ah_tl(AH a) {
+    const double t = (a.d[0] + a.d[1] + a.d[2]) / 3.0;
+    a.d[0] -= t;
+    a.d[1] -= t;
+    a.d[2] -= t;
+    return a;
+}
+IPG_HD AH operator+(const AH& a, const AH& b) {
+    AH c;
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        c.d[k] = a.d[k] + b.d[k];
+        c.o[k] = a.o[k] + b.o[k];
+    }
+    return c;
+}
+IPG_HD AH operator-(const AH& a, const AH& b) {
+    AH c;
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        c.d[k] = a.d[k] - b.d[k];
+        c.o[k] = a.o[k] - b.o[k];
+    }
+    return c;
+}
+// (1 + X + X^2/2) with X = i c E, E Hermitian: X^2 = -c^2 E^2
+IPG_HD M3 taylor2(double c, const H3& e) {
+    const double h = 0.5 * c * c;
+    M3 m;
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+        const int k = (i + 1) % 3, l = (i + 2) % 3;
+        const cd ok = h_off(e, i, k), ol = h_off(e, i, l);
+        const double sq = e.d[i] * e.d[i] + (ok.r * ok.r + ok.i * ok.i) + (ol.r * ol.r + ol.i * ol.i);
+        m.e[4 * i] = cd{1. - h * sq, c * e.d[i]};
+    }
+#pragma unroll
+    for (int q = 0; q < 3; q++) {
+        const int i = q == 2 ? 1 : 0, j = q == 0 ? 1 : 2, n = 3 - i - j;
+        const cd sq = e.o[q] * (e.d[i] + e.d[j]) + h_off(e, i, n) * h_off(e, n, j);
+        m.e[3 * i + j] = cd{-h * sq.r - c * e.o[q].i, -h * sq.i + c * e.o[q].r};
+        m.e[3 * j + i] = cd{-h * sq.r + c * e.o[q].i, h * sq.i + c * e.o[q].r};
+    }
+    return m;
+}
+
 // the stored (upper-triangle) form of a matrix, expanded again
 IPG_HD M3 herm_part(const M3& m) {
     M3 h;
