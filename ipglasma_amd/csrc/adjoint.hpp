@@ -166,6 +166,122 @@ IPG_HD void u_adj(const M3& U, const M3& E, double kappa, const M3& Yb, M3& Ub, 
     Eb = Eb + cscale(cd{0., -kappa}, Xb);
 }
 
+// ---- the leapfrog step in reverse, gathered per site -------------------------------
+// The cotangents a site's own fields receive, from the sites of its stencil
+// (the same sums as e_adj and pi_adj scatter).  Z1, Z2 are the traceless
+// Hermitian cotangents of E1', E2' and bb = (dtau/tau) of pi''s.  With
+// a = tau dtau / (2 g^2), the plaquettes of E' have the cotangents
+//   U12 = Ux Uy(+x) Ux(+y)^+ Uy^+             -2ia (Z1 - Z2)
+//   U1m2 = Ux Uy(+x-y)^+ Ux(-y)^+ Uy(-y)      -2ia Z1
+//   U2m1 = Uy Ux(-x+y)^+ Uy(-x)^+ Ux(-x)      -2ia Z2
+// and a link U_x(t) enters three of each through the loop above it (corners t,
+// t+x, t+y) and three through the loop below it (corners t-y, t+x-y, t).  The
+// lattice is clamped: at its edges a site is its own neighbour, so some
+// sources are missing and others come twice (the weights and extra terms).
+// The y link is the x link with the axes exchanged (x <-> y, Z1 <-> Z2), so
+// one code serves both: F has the site's coordinates p along and q across the
+// link, N, and uf, uo (links along and across), zf, zo, ph, bb at the clamped
+// offset (dp, dq) from it.
+
+// keeps the scheduler from having every factor of a sum loaded at once
+IPG_HD void adj_fence() {
+#ifdef __HIP_DEVICE_COMPILE__
+    __builtin_amdgcn_sched_barrier(0);
+#endif
+}
+// the loop above the link, in units of -2ia.  First the sources every site has
+// (weights 0 where an edge takes one away), then, on the edges, the sources
+// that are there twice: the same body with other sites and weights, so that
+// the code stays small (the instruction cache holds 64 KB).
+template <class F>
+IPG_HD M3 adj_link_above(const F& f) {
+    const int N = f.N;
+    M3 r = m_zero();
+#pragma unroll 1
+    for (int rep = 0; rep < 3; rep++) {
+        // 1: the site is its own neighbour below (U1m2 of the site itself), 2:
+        // its own neighbour behind (U2m1 of the site itself)
+        if ((rep == 1 && f.q != 0) || (rep == 2 && f.p != 0)) continue;
+        const int l = rep == 1 ? 0 : 1, m = rep == 2 ? 0 : 1;
+        const double wd = rep == 0 ? 1. : 0., wz = rep == 1 || (rep == 0 && f.q < N - 1) ? 1. : 0.;
+        const double wo = rep == 2 || (rep == 0 && f.p < N - 1) ? 1. : 0.;
+        const M3 G = mul_bd(f.uf(0, l), f.uo(m, 0));
+        const M3 U = f.uo(0, 0);
+        const M3 T = mac_mh(mul_h(wd * (f.zf(0, 0) - f.zo(0, 0)), U), U, -wz * f.zf(0, l));
+        r = mac(r, T, G);
+        adj_fence();
+        r = mac(r, U, mul_mh(G, wo * f.zo(m, 0)));
+        adj_fence();
+    }
+    return r;
+}
+// the loop below the link, in units of -2ia
+template <class F>
+IPG_HD M3 adj_link_below(const F& f) {
+    const int N = f.N;
+    M3 r = m_zero();
+#pragma unroll 1
+    for (int rep = 0; rep < 2; rep++) {
+        // 1: the site is its own neighbour above (U12 and U2m1 of its own row)
+        if (rep == 1 && f.q != N - 1) continue;
+        const int l = rep == 0 ? -1 : 0;
+        const double wc = rep == 0 ? 1. : 0., wb = rep == 1 || f.q > 0 ? 1. : 0., we = f.p < N - 1 ? wb : 0.;
+        const M3 U = f.uo(0, l), u = f.uf(0, l);
+        // Z U^+ - U^+ D = (U Z - D U)^+
+        const M3 T = mac_mh(mul_h(-wb * (f.zf(0, l) - f.zo(0, l)), U), U, wc * f.zf(0, 0));
+        const M3 X = mac_ad(mul_ad(T, u), U, mul_mh(u, -we * f.zo(1, l)));
+        r = mac(r, X, f.uo(1, l));
+        adj_fence();
+        if (f.p == 0 && wb != 0.) {
+            const M3 V = f.uo(0, l);
+            r = r - mul_ad(V, f.uf(0, l)) * mul_h(f.zo(0, l), V);
+        }
+        adj_fence();
+    }
+    return r;
+}
+// bb of the sites whose neighbour against the link's direction is this one
+template <class F>
+IPG_HD H3 adj_bb_sum(const F& f) {
+    const double w1 = f.p < f.N - 1 ? 1. : 0., w0 = f.p == 0 ? 1. : 0.;
+    return w1 * f.bb(1, 0) + w0 * f.bb(0, 0);
+}
+// bb + the cotangent of phi~ from the commutator of E', k = dtau/tau
+template <class F>
+IPG_HD H3 adj_q(const F& f, int dp, double k) {
+    return f.bb(dp, 0) + herm_mi(k, commutator(f.zf(dp, 0), f.ph(dp, 0)));
+}
+// the link's share of the commutator of E' and of the pi' stencil
+template <class F>
+IPG_HD M3 adj_link_phi(const F& f, double k) {
+    const M3 u = f.uf(0, 0);
+    const M3 a = mul_mh(mul_h(adj_q(f, 0, k), u), f.ph(1, 0));
+    adj_fence();
+    return 2. * (a + mul_h(f.ph(0, 0), mul_mh(u, adj_bb_sum(f))));
+}
+// phi's share through the links of this direction (without -4 bb)
+template <class F>
+IPG_HD H3 adj_phi_dir(const F& f, double k) {
+    const M3 u = f.uf(0, 0);
+    const H3 tx = herm_mul(u, mul_hd(f.ph(1, 0), u));
+    H3 r = herm_mi(k, commutator(tx, f.zf(0, 0))) + herm_mul(u, mul_hd(adj_bb_sum(f), u));
+    adj_fence();
+    if (f.p > 0) {
+        const M3 v = f.uf(-1, 0);
+        r = r + herm_mul_ad(v, mul_h(adj_q(f, -1, k), v));
+    }
+    if (f.p == f.N - 1) r = r + herm_mul_ad(u, mul_h(adj_q(f, 0, k), u));
+    return r;
+}
+// U' = M(E') U in reverse (u_adj) with Hermitian E': M^+ Yb, and e + TL of what
+// E' receives
+IPG_HD M3 adj_link_update(const M3& U, const H3& E, double kappa, const M3& Yb, const H3& e, H3& z) {
+    const M3 Mb = mul_bd(Yb, U);
+    // -i kappa Xb, Hermitian part: (-i kappa/2)(Mb - Mb^+) - (kappa^2/4) {Mb + Mb^+, E}
+    z = h_traceless((e + herm_mi(0.5 * kappa, ah_of(Mb))) - (0.25 * kappa * kappa) * anticommutator(two_herm(Mb), E));
+    return mul_ad(taylor2(kappa, E), Yb);
+}
+
 // ---- T^tautau at one site (lattice units, before the a^-4) ----------------------------
 // e1, e1py = E1(s), E1(s+y); e2, e2px = E2(s), E2(s+x); pi at s, s+x, s+y,
 // s+x+y; links for the plaquette and the phi gradients; phi at s, s+x, s+y,

@@ -1188,7 +1188,7 @@ struct Engine {
     static size_t adj_evolution_doubles(const EvDesc& d, int K) {
         const int T = d.itmax - 1;
         const size_t nslot = 1 + (size_t)(T / K + 1) + (size_t)K + 1 + 1;
-        return nslot * 72 * (size_t)d.S + (2 * IPG_PEND_PLANES + 108 + 10) * (size_t)d.S + 16;
+        return nslot * 72 * (size_t)d.S + (2 * IPG_COT_PLANES + 108 + 10) * (size_t)d.S + 16;
     }
     // doubles the reverse mode to rho needs beyond the evolution part: V_A,
     // V_B and the link and D cotangents (2 x 18 planes each), and the
@@ -1371,7 +1371,7 @@ struct Engine {
         const int K = Kfix > 0 ? Kfix : adj_interval(d, 0);
         last_K = K;
         const int nck = T / K + 1;
-        const size_t slot = 72 * (size_t)S, pend = IPG_PEND_PLANES * (size_t)S, cset = 108 * (size_t)S;
+        const size_t slot = 72 * (size_t)S, pend = IPG_COT_PLANES * (size_t)S, cset = 108 * (size_t)S;
         rho_grad = nullptr;
         rho_grad_n = 0;
         const size_t need = adj_evolution_doubles(d, K);
@@ -1384,7 +1384,7 @@ struct Engine {
         double* s_ck = s_init + slot;                 // nck checkpoints
         double* s_seg = s_ck + (size_t)nck * slot;    // K + 1 segment states
         double* s_T = s_seg + (size_t)(K + 1) * slot;
-        double* cA = s_T + slot;     // pending cotangent sets
+        double* cA = s_T + slot;     // cotangent sets
         double* cB = cA + pend;
         double* c0 = cB + pend;      // compact cotangents of the tau = 0 fields
         double* tb = c0 + cset;      // cotangents of the ten T^{mu nu} planes at itmax
@@ -1536,24 +1536,41 @@ struct Engine {
             ipg_adj_tmunu(d_adesc, S, sT, itm, tb, cA, st);
         }
         double *cin = cA, *cout = cB;
-        // the reverse step's kernel split (the tuner's choice)
+        // the gather of a step and the local updates of the step before it as
+        // one kernel or as two (the tuner's choice)
         const std::string rkey = "adj_step_kernels/N=" + std::to_string(d.N);
+        bool mid = false;  // the local updates of the next step to reverse are done
         for (int k = nck - 1; k >= 0; k--) {
             const int s0 = k * K, s1 = std::min(s0 + K, T);
             if (s1 <= s0) continue;
             const double* x0 = s_ck + (size_t)k * slot;
             if (K > 1)
                 for (int it = s0 + 1; it <= s1; it++) ipg_launch_step(d_rdesc + (it - 1), 1, nb, it, st, sv);
+            // the state after step it (s0 <= it <= s1); K = 1: the next stored state
+            auto state = [&](int it) -> const double* {
+                if (it == s0) return x0;
+                return K > 1 ? s_seg + (size_t)(it - s0) * slot : s_ck + (size_t)it * slot;
+            };
             for (int it = s1; it > s0; it--) {
-                const double* xb = it - 1 == s0 ? x0 : s_seg + (size_t)(it - 1 - s0) * slot;
-                // K = 1: the state after the step is the next stored state
-                const double* xa = K > 1 ? s_seg + (size_t)(it - s0) * slot : s_ck + (size_t)it * slot;
-                bool rm = false;
-                const int rv = g_tuner.pick(rkey, 3, &rm);
-                hipEvent_t ra = nullptr, rb = nullptr;
-                if (timed_begin(rkey, rv, rm, &ra, &rb)) (void)hipEventRecord(ra, st);
-                ipg_adj_step(d_adesc, S, xb, xa, it, cin, cout, st, rv);
-                if (rb) (void)hipEventRecord(rb, st);
+                if (!mid) ipg_adj_local(d_adesc, S, state(it - 1), state(it), it, cin, st);
+                // the state before step it - 1, where it is stored or recomputed
+                const double* xp = it - 1 > s0 ? state(it - 2) : (tape && it > 1 ? s_ck + (size_t)(it - 2) * slot : nullptr);
+                if (xp) {
+                    bool rm = false;
+                    const int rv = g_tuner.pick(rkey, 2, &rm);
+                    hipEvent_t ra = nullptr, rb = nullptr;
+                    if (timed_begin(rkey, rv, rm, &ra, &rb)) (void)hipEventRecord(ra, st);
+                    if (rv == 0) {
+                        ipg_adj_gather(d_adesc, S, state(it - 1), xp, it, cin, cout, st);
+                    } else {
+                        ipg_adj_gather(d_adesc, S, state(it - 1), nullptr, it, cin, cout, st);
+                        ipg_adj_local(d_adesc, S, xp, state(it - 1), it - 1, cout, st);
+                    }
+                    if (rb) (void)hipEventRecord(rb, st);
+                } else {
+                    ipg_adj_gather(d_adesc, S, state(it - 1), nullptr, it, cin, cout, st);
+                }
+                mid = xp != nullptr;
                 std::swap(cin, cout);
             }
         }

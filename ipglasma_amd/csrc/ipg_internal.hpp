@@ -88,25 +88,26 @@ void ipg_launch_pi_init(const EvDesc* d_evs, int nev, int nblk, hipStream_t st);
 void ipg_launch_zero_fields(const EvDesc* d_evs, int nev, int nblk, hipStream_t st);
 void ipg_launch_rho_normals(const EvDesc* d_evs, int nucleus, int k, double* d_out, hipStream_t st);
 
-// reverse mode of dE/deta through the leapfrog (one event, evs[0]); the
-// step's cotangents travel in pending sets of IPG_PEND_PLANES planes (own
-// cotangents plus what each site sends to its neighbours), the loss fills
-// one (zeroed by the caller), the kick turns the last into a compact set of
-// 108 planes
-#define IPG_PEND_PLANES 252
+// reverse mode of dE/deta through the leapfrog (one event, evs[0]); a
+// cotangent set has IPG_COT_PLANES planes; the loss fills one (zeroed by the
+// caller), the kick turns the last into a compact set of 108 planes
+#define IPG_COT_PLANES 72
 void ipg_adj_state_save(const EvDesc* d_evs, long long S, int parity, double* slot, hipStream_t st);
 void ipg_adj_state_load(const EvDesc* d_evs, long long S, int parity, const double* slot, hipStream_t st);
 void ipg_adj_zero(double* p, long long n, hipStream_t st);
 void ipg_adj_loss(const EvDesc* d_evs, long long S, const double* xs, int it, double yb, double* cout,
                   hipStream_t st);
-// variant 0: three kernels (own-field planes, link outboxes, phi outboxes),
-// 1: one kernel running the three passes per site with the partial sums of
-// the link cotangents in LDS, 2: the first kernel, then passes 2 and 3 as
-// one with those sums in LDS (the same results)
-void ipg_adj_step(const EvDesc* d_evs, long long S, const double* xb, const double* xa, int it, const double* cin,
-                  double* cout, hipStream_t st, int variant = 0);
+// the site-local updates of step it in reverse, in place (xb, xa: the states
+// before and after it): the state's cotangents -> the step's middle set
+void ipg_adj_local(const EvDesc* d_evs, long long S, const double* xb, const double* xa, int it, double* c,
+                   hipStream_t st);
+// the gather of step it: its middle set cin -> the cotangents of the state xb
+// before it; with xp (the state before step it - 1) also the local updates of
+// step it - 1: -> its middle set
+void ipg_adj_gather(const EvDesc* d_evs, long long S, const double* xb, const double* xp, int it, const double* cin,
+                    double* cout, hipStream_t st);
 // T^{mu nu} at it in reverse: tb[10][S] cotangents of the stored components,
-// field cotangents of the state xs into a zeroed pending set
+// field cotangents of the state xs into a zeroed cotangent set
 void ipg_adj_tmunu(const EvDesc* d_evs, long long S, const double* xs, int it, const double* tb, double* pout,
                    hipStream_t st);
 // d eps_2 / dT at it (after ipg_launch_landau of the same it) into tb[10][S]

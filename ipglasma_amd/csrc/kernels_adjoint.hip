@@ -7,23 +7,17 @@
 // recomputes segment by segment from checkpoints (every K = ceil(sqrt(T))
 // steps).
 //
-// No atomics in the step: every site writes the cotangents of its own fields
-// ("self") and, per neighbour offset, the cotangent it sends to that
-// neighbour ("outbox"); the next reverse step gathers the outboxes of the
-// sites whose clamped neighbour it is.  One step runs as three site-parallel
-// passes (local updates; the three plaquettes of E'; the commutators of E'
-// and the pi' stencil) so that few matrices are live at a time.
+// No atomics in the step: every site gathers the cotangents of its own fields
+// from its stencil (adj_link_above, adj_link_below, adj_link_phi,
+// adj_phi_dir of adjoint.hpp).  A reverse step is a gather (the plaquettes and
+// commutators of E' and the pi' stencil) followed by the site-local updates of
+// the step before it (the link update, phi'), so one kernel does both.
 //
 // A state slot is 72 planes of S doubles: U_x, U_y (18 each, full complex),
-// E1, E2, phi, pi (9 each, Hermitian storage).  A compact cotangent set is
-// 108 planes: U_x, U_y, E1, E2, phi, pi, all full complex (18 each).  A
-// pending set is kPend planes:
-//   self     U_x, U_y (18 each), E1, E2, phi, pi (9 each, Hermitian)
-//   outbox   U_x to (0,+1) (0,-1) (-1,+1) (-1,0)   4 x 18
-//            U_y to (+1,0) (+1,-1) (0,-1) (-1,0)   4 x 18
-//            phi to (+1,0) (0,+1) (-1,0) (0,-1)    4 x 9 (Hermitian)
-// The cotangents of E, phi and pi are used only through their Hermitian
-// part, so self and outbox keep that part.
+// E1, E2, phi, pi (9 each, Hermitian storage).  A cotangent set has the same
+// 72 planes: the cotangents of E, phi and pi are used only through their
+// Hermitian part.  A compact cotangent set, what the initial conditions take,
+// is 108 planes: U_x, U_y, E1, E2, phi, pi, all full complex (18 each).
 #include "adjoint.hpp"
 #include "ipg_device.hpp"
 #include "ipg_internal.hpp"
@@ -46,10 +40,9 @@ __device__ __forceinline__ Slot slot_of(const double* base, size_t S) {
 // cotangent set: field f (0 Ux, 1 Uy, 2 E1, 3 E2, 4 phi, 5 pi)
 __device__ __forceinline__ double* cot(double* base, size_t S, int f) { return base + (size_t)f * 18 * S; }
 
-// pending set planes
+// planes of a cotangent set
 constexpr int kPU1 = 0, kPU2 = 18, kPE1 = 36, kPE2 = 45, kPPh = 54, kPPi = 63;
-constexpr int kPOx = 72, kPOy = 144, kPOph = 216;
-static_assert(kPOph + 36 == IPG_PEND_PLANES, "pending set layout");
+static_assert(kPPi + 9 == IPG_COT_PLANES, "cotangent set layout");
 
 __device__ __forceinline__ void atomic_add_m3(double* f, size_t S, size_t s, const M3& m) {
 #pragma unroll
@@ -58,14 +51,6 @@ __device__ __forceinline__ void atomic_add_m3(double* f, size_t S, size_t s, con
         atomicAdd(f + (2 * k + 1) * S + s, m.e[k].i);
     }
 }
-__device__ __forceinline__ void add_m3(double* f, size_t S, size_t s, const M3& m) {
-#pragma unroll
-    for (int k = 0; k < 9; k++) {
-        f[(2 * k) * S + s] += m.e[k].r;
-        f[(2 * k + 1) * S + s] += m.e[k].i;
-    }
-}
-
 // adds hproj(m) to a Hermitian-storage plane group
 __device__ __forceinline__ void atomic_add_h(double* f, size_t S, size_t s, const M3& m) {
     const M3 h = hproj(m);
@@ -79,61 +64,6 @@ __device__ __forceinline__ void atomic_add_h(double* f, size_t S, size_t s, cons
     atomicAdd(f + 7 * S + s, h.e[5].r);
     atomicAdd(f + 8 * S + s, h.e[5].i);
 }
-__device__ __forceinline__ void add_h(double* f, size_t S, size_t s, const M3& h) {
-    sth<true>(f, S, s, ldh<true>(f, S, s) + h);
-}
-
-// The sites u along one axis whose clamped neighbour clamp(u + d) is t: one
-// in the interior, two or none at the edges.
-struct Src {
-    int a, b, n;
-};
-__device__ __forceinline__ Src srcs(int t, int d, int N) {
-    if (d == 0) return Src{t, t, 1};
-    if (d > 0) return t == N - 1 ? Src{t - 1, t, 2} : (t >= 1 ? Src{t - 1, t - 1, 1} : Src{0, 0, 0});
-    return t == 0 ? Src{1, 0, 2} : (t <= N - 2 ? Src{t + 1, t + 1, 1} : Src{0, 0, 0});
-}
-// what site (i, j) receives through one outbox offset (di, dj)
-template <bool HERM>
-__device__ __forceinline__ M3 gather(const double* f, size_t S, int N, int i, int j, int di, int dj) {
-    const Src a = srcs(i, di, N), b = srcs(j, dj, N);
-    M3 r = m_zero();
-    for (int p = 0; p < a.n; p++) {
-        const int si = p ? a.b : a.a;
-        for (int q = 0; q < b.n; q++) {
-            const int sj = q ? b.b : b.a;
-            const size_t u = (size_t)si * N + sj;
-            r = r + (HERM ? ldh<true>(f, S, u) : ldm<true>(f, S, u));
-        }
-    }
-    return r;
-}
-// total cotangents of U_x, U_y and phi at (i, j) = s in a pending set
-__device__ __forceinline__ M3 cin_ux(const double* P, size_t S, int N, int i, int j, size_t s) {
-    M3 r = ldm<true>(P + kPU1 * S, S, s);
-    r = r + gather<false>(P + (kPOx + 0) * S, S, N, i, j, 0, 1);
-    r = r + gather<false>(P + (kPOx + 18) * S, S, N, i, j, 0, -1);
-    r = r + gather<false>(P + (kPOx + 36) * S, S, N, i, j, -1, 1);
-    r = r + gather<false>(P + (kPOx + 54) * S, S, N, i, j, -1, 0);
-    return r;
-}
-__device__ __forceinline__ M3 cin_uy(const double* P, size_t S, int N, int i, int j, size_t s) {
-    M3 r = ldm<true>(P + kPU2 * S, S, s);
-    r = r + gather<false>(P + (kPOy + 0) * S, S, N, i, j, 1, 0);
-    r = r + gather<false>(P + (kPOy + 18) * S, S, N, i, j, 1, -1);
-    r = r + gather<false>(P + (kPOy + 36) * S, S, N, i, j, 0, -1);
-    r = r + gather<false>(P + (kPOy + 54) * S, S, N, i, j, -1, 0);
-    return r;
-}
-__device__ __forceinline__ M3 cin_ph(const double* P, size_t S, int N, int i, int j, size_t s) {
-    M3 r = ldh<true>(P + kPPh * S, S, s);
-    r = r + gather<true>(P + (kPOph + 0) * S, S, N, i, j, 1, 0);
-    r = r + gather<true>(P + (kPOph + 9) * S, S, N, i, j, 0, 1);
-    r = r + gather<true>(P + (kPOph + 18) * S, S, N, i, j, -1, 0);
-    r = r + gather<true>(P + (kPOph + 27) * S, S, N, i, j, 0, -1);
-    return r;
-}
-
 // the site of this thread in a launch of pad8(ceil(S / IPG_BLOCK)) blocks:
 // the XCD-aware block order of the forward kernels (xcd_remap), so that the
 // blocks of neighbouring lattice rows run on one XCD and share its L2
@@ -192,7 +122,7 @@ __global__ __launch_bounds__(IPG_BLOCK) void k_zero(double* __restrict__ p, long
 }
 
 // ---- loss: dL/dT^tautau(s) = tau_fm hbarc / a^2 for every site --------------------
-// into the own-field planes of a zeroed pending set
+// into a zeroed cotangent set
 __global__ __launch_bounds__(IPG_BLOCK) void k_adj_loss(const EvDesc* __restrict__ evs, const double* __restrict__ xs,
                                                        int it, double yb, double* __restrict__ cout) {
     const EvDesc& ev = evs[0];
@@ -250,7 +180,7 @@ __global__ __launch_bounds__(IPG_BLOCK) void k_adj_loss(const EvDesc* __restrict
 // ---- T^{mu nu} at itmax in reverse (Evolution.cpp:659-1246) -----------------------
 // tb: cotangents of the ten stored components (T's order, after the a^-4,
 // a^-5, a^-6 scalings) at every site; the cotangents of the fields of the
-// state xs go into the own-field planes of a zeroed pending set (atomics:
+// state xs go into a zeroed cotangent set (atomics:
 // each site's terms reach up to two sites away).  Three passes as the
 // forward's: diagonal components with T^{tau eta} and T^{xy}; the clovers of
 // T^{tau x}, T^{tau y}, T^{x eta}, T^{y eta}; their pi and E pi parts.
@@ -573,301 +503,248 @@ __global__ __launch_bounds__(IPG_BLOCK) void k_adj_fill_tb(long long S, const do
 }
 
 // ---- one leapfrog step in reverse ------------------------------------------------------
-// xb: state before the step, xa: state after; pin: pending cotangents of the
-// state after; pout: pending cotangents of the state before (every plane is
-// written: pass 1 the own-field planes, pass 2 the link outboxes, pass 3 the
-// phi outboxes)
+// Two kinds of cotangent set pass from kernel to kernel: a full one (the
+// cotangents of a state) and, after the site-local updates of step it, a
+// middle one (M^+ U'b in the place of U, Z_i = TL(E_i'b) of E, phi'b and pi'b),
+// from which the step's gather makes the full set of the state before it.
 
-// pass 1, site-local: U' = M(E') U, phi' = phi + (tau + dtau/2) dtau pi',
-// and the traceless part taken by E'.  Leaves in pout: the U cotangents from
-// the link update, Z_i = TL(E_i'b) (the own E_i cotangent), phi'b and pi'b.
-__device__ __forceinline__ void adj_local_site(const EvDesc& ev, long long s, const double* __restrict__ xb,
-                                               const double* __restrict__ xa, int it, const double* __restrict__ pin,
-                                               double* __restrict__ pout) {
+// The gather's stencil is staged in LDS: of a block's 64 sites the rows i and
+// i+1 (117 planes, each with the sites past the block's ends: 66 values),
+// loaded once with every load in flight before anything is computed.  Row i-1
+// is read by one role each and comes from memory.
+constexpr int kRoleSites = 64;  // sites of a block: one wavefront per role
+constexpr int kGUx = 0, kGUy = 18, kGZ1 = 36, kGZ2 = 45, kGPh = 54, kGPi = 63;  // row i
+constexpr int kGUyP = 72, kGZ2P = 90, kGPhP = 99, kGPiP = 108;                 // row i+1
+constexpr int kGPlanes = 117;
+typedef double GRow[kRoleSites + 2];
+__device__ __forceinline__ M3 row_m(const GRow* f, int q) {
+    M3 m;
+#pragma unroll
+    for (int k = 0; k < 9; k++) m.e[k] = cd{f[2 * k][q], f[2 * k + 1][q]};
+    return m;
+}
+__device__ __forceinline__ H3 row_h(const GRow* f, int q) {
+    H3 h;
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        h.d[k] = f[k][q];
+        h.o[k] = cd{f[3 + 2 * k][q], f[4 + 2 * k][q]};
+    }
+    return h;
+}
+template <int NP>
+__device__ __forceinline__ void stage_rows(GRow* to, const double* f, size_t S, size_t s, int lane) {
+    double v[NP];
+    const unsigned ob = lane_offset<false>(s);
+#pragma unroll
+    for (int k = 0; k < NP; k++) v[k] = gld(f, k * S, ob);
+#pragma unroll
+    for (int k = 0; k < NP; k++) to[k][lane + 1] = v[k];
+}
+
+// fields of a site's stencil at the clamped offset (dp, dq) along and across
+// the link direction dir, a run-time choice, so that both directions run the
+// same code
+struct StepAcc {
+    const GRow* st;
+    const double *Ux, *Uy, *Z1, *Z2, *Ph, *Pi;
+    size_t S, sm;  // sm: the site of row i-1 (clamped)
+    int N, dir, p, q, lane, j;
+    double k;
+    __device__ __forceinline__ int row(int dp, int dq) const { return dir ? dq : dp; }
+    __device__ __forceinline__ int dcol(int dp, int dq) const {
+        const int d = dir ? dp : dq;
+        return d > 0 ? (j < N - 1 ? 1 : 0) : d < 0 ? (j > 0 ? -1 : 0) : 0;
+    }
+    // f: planes in row i, fp: in row i+1 (negative: not staged, never asked for)
+    __device__ __forceinline__ M3 um(int f, int fp, const double* g, int dp, int dq) const {
+        const int r = row(dp, dq), c = dcol(dp, dq);
+        if (r < 0) return ldm<true>(g, S, sm + c);
+        return row_m(st + (r > 0 ? fp : f), lane + 1 + c);
+    }
+    __device__ __forceinline__ H3 hm(int f, int fp, const double* g, int dp, int dq) const {
+        const int r = row(dp, dq), c = dcol(dp, dq);
+        if (r < 0) return ldh3<true>(g, S, sm + c);
+        return row_h(st + (r > 0 ? fp : f), lane + 1 + c);
+    }
+    // along x: U_x is staged in row i alone; uf is asked for at dp <= 0, so
+    // row i+1 is uf of the y direction (U_y) or uo of the x direction (U_y)
+    __device__ __forceinline__ M3 uf(int dp, int dq) const {
+        return um(dir ? kGUy : kGUx, kGUyP, dir ? Uy : Ux, dp, dq);
+    }
+    __device__ __forceinline__ M3 uo(int dp, int dq) const {
+        return um(dir ? kGUx : kGUy, kGUyP, dir ? Ux : Uy, dp, dq);
+    }
+    __device__ __forceinline__ H3 zf(int dp, int dq) const {
+        return hm(dir ? kGZ2 : kGZ1, kGZ2P, dir ? Z2 : Z1, dp, dq);
+    }
+    __device__ __forceinline__ H3 zo(int dp, int dq) const {
+        return hm(dir ? kGZ1 : kGZ2, kGZ2P, dir ? Z1 : Z2, dp, dq);
+    }
+    __device__ __forceinline__ H3 ph(int dp, int dq) const { return hm(kGPh, kGPhP, Ph, dp, dq); }
+    __device__ __forceinline__ H3 bb(int dp, int dq) const { return k * hm(kGPi, kGPiP, Pi, dp, dq); }
+};
+
+// The gather of step it and (FUSE) the site-local updates of step it - 1.  xb:
+// state before step it, xp (FUSE): state before step it - 1; pin: the middle
+// set of step it; pout: the middle set of step it - 1 (FUSE) or the full set of
+// the state before step it.  A block takes 64 sites with four wavefronts, each
+// in a role: phi and pi; U_x and E1; U_y and E2; the loops below both links
+// (handed over through LDS), ~1100-1300 FP64 multiply-adds a lane each.
+// FP64 issue and the latency of dependent products at two waves per SIMD bound
+// it (243 planes of unique traffic: 510 MB at N = 512, ~105 us as a copy).
+// Measured per step, N = 192 / 256 / 512: what each site sends to its
+// neighbours written out and gathered by the next step (252 planes a set) 59 /
+// 82 / 368 us; this gather with every role loading its own matrices 39 / 53 /
+// 202 us; staged 34 / 43 / 164 us; with products as multiply-add chains 30 /
+// 40 / 152 us.
+template <bool FUSE>
+__global__ __launch_bounds__(4 * kRoleSites, 2) void k_adj_gather(const EvDesc* __restrict__ evs,
+                                                                 const double* __restrict__ xb,
+                                                                 const double* __restrict__ xp, int it,
+                                                                 const double* __restrict__ pin,
+                                                                 double* __restrict__ pout) {
+    __shared__ GRow stage[kGPlanes];
+    __shared__ double low[2][18][kRoleSites];
+    const EvDesc& ev = evs[0];
     const size_t S = ev.S;
-    const int N = ev.N, i = (int)(s / N), j = (int)(s - (long long)i * N);
+    const int lb = xcd_remap((int)blockIdx.x, (int)gridDim.x);
+    // N is a multiple of 16, S of 256: a block is full or past the end
+    if ((size_t)lb * kRoleSites >= S) return;
+    const int lane = (int)(threadIdx.x & 63);
+    const int role = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const size_t s0 = (size_t)lb * kRoleSites, s = s0 + lane;
+    const int N = ev.N, i = (int)s / N, j = (int)s - i * N;
+    const double dt = ev.dtau, tau = it * dt, k = dt / tau;
+    const Slot B = slot_of(xb, S);
+    const double* const z1 = pin + kPE1 * S;
+    const double* const z2 = pin + kPE2 * S;
+    const double* const pib_ = pin + kPPi * S;
+    {
+        const size_t pX = (size_t)min(i + 1, N - 1) * N + j;
+        if (role == 0) {
+            stage_rows<18>(stage + kGUx, B.Ux, S, s, lane);
+            stage_rows<9>(stage + kGPh, B.phi, S, s, lane);
+        } else if (role == 1) {
+            stage_rows<18>(stage + kGUy, B.Uy, S, s, lane);
+            stage_rows<9>(stage + kGPi, pib_, S, s, lane);
+            stage_rows<9>(stage + kGZ2P, z2, S, pX, lane);
+        } else if (role == 2) {
+            stage_rows<18>(stage + kGUyP, B.Uy, S, pX, lane);
+            stage_rows<9>(stage + kGPhP, B.phi, S, pX, lane);
+        } else {
+            stage_rows<9>(stage + kGZ1, z1, S, s, lane);
+            stage_rows<9>(stage + kGZ2, z2, S, s, lane);
+            stage_rows<9>(stage + kGPiP, pib_, S, pX, lane);
+        }
+        // the sites past the block's ends: plane t / 2, left and right
+        const int t = (int)threadIdx.x;
+        if (t < 2 * kGPlanes) {
+            const int pl = t >> 1, right = t & 1;
+            const int se = (int)s0 + (right ? kRoleSites - 1 : 0), ie = se / N, je = se - ie * N;
+            const int jn = right ? min(je + 1, N - 1) : max(je - 1, 0);
+            const size_t q = (size_t)(pl < kGUyP ? ie : min(ie + 1, N - 1)) * N + jn;
+            const double* f = pl < kGUy    ? B.Ux + pl * S
+                              : pl < kGZ1  ? B.Uy + (pl - kGUy) * S
+                              : pl < kGZ2  ? z1 + (pl - kGZ1) * S
+                              : pl < kGPh  ? z2 + (pl - kGZ2) * S
+                              : pl < kGPi  ? B.phi + (pl - kGPh) * S
+                              : pl < kGUyP ? pib_ + (pl - kGPi) * S
+                              : pl < kGZ2P ? B.Uy + (pl - kGUyP) * S
+                              : pl < kGPhP ? z2 + (pl - kGZ2P) * S
+                              : pl < kGPiP ? B.phi + (pl - kGPhP) * S
+                                           : pib_ + (pl - kGPiP) * S;
+            stage[pl][right ? kRoleSites + 1 : 0] = f[q];
+        }
+    }
+    StepAcc f{stage, B.Ux, B.Uy, z1, z2, B.phi, pib_, S, (size_t)max(i - 1, 0) * N + j, N, 0, i, j, lane, j, k};
+    __syncthreads();
+    if (role == 0) {
+        const H3 pib = row_h(stage + kGPi, lane + 1);
+        H3 r = ldh3<true>(pin + kPPh * S, S, s) + (-4. * k) * pib;
+#pragma unroll 1
+        for (int dir = 0; dir < 2; dir++) {
+            f.dir = dir;
+            f.p = dir ? j : i;
+            f.q = dir ? i : j;
+            r = r + adj_phi_dir(f, k);
+        }
+        sth3<true>(pout + kPPh * S, S, s, r);
+        sth3<true>(pout + kPPi * S, S, s, FUSE ? pib + (((tau - dt) + dt / 2.) * dt) * r : pib);
+        __syncthreads();
+    } else if (role == 3) {
+        const double c = -tau * dt / (ev.g * ev.g);
+#pragma unroll 1
+        for (int dir = 0; dir < 2; dir++) {
+            f.dir = dir;
+            f.p = dir ? j : i;
+            f.q = dir ? i : j;
+            const M3 m = mul_i(c, adj_link_below(f));
+#pragma unroll
+            for (int q = 0; q < 9; q++) {
+                low[dir][2 * q][lane] = m.e[q].r;
+                low[dir][2 * q + 1][lane] = m.e[q].i;
+            }
+        }
+        __syncthreads();
+    } else {
+        const int dir = role - 1;
+        const double g = ev.g;
+        f.dir = dir;
+        f.p = dir ? j : i;
+        f.q = dir ? i : j;
+        M3 r = mul_i(-tau * dt / (g * g), adj_link_above(f));
+        r = r + adj_link_phi(f, k);
+        adj_fence();
+        r = r + ldm<true>(pin + (dir ? kPU2 : kPU1) * S, S, s);
+        const H3 z = f.zf(0, 0);
+        __syncthreads();
+#pragma unroll
+        for (int c = 0; c < 9; c++) r.e[c] = r.e[c] + cd{low[dir][2 * c][lane], low[dir][2 * c + 1][lane]};
+        double* cu = pout + (dir ? kPU2 : kPU1) * S;
+        double* ce = pout + (dir ? kPE2 : kPE1) * S;
+        if (FUSE) {
+            const Slot P = slot_of(xp, S);
+            const double kappa = g * g * dt / ((tau - dt) + dt / 2.);
+            H3 zp;
+            const M3 ub = adj_link_update(ldm<true>(dir ? P.Uy : P.Ux, S, s), ldh3<true>(dir ? B.E2 : B.E1, S, s),
+                                          kappa, r, z, zp);
+            stm<true>(cu, S, s, ub);
+            sth3<true>(ce, S, s, zp);
+        } else {
+            stm<true>(cu, S, s, r);
+            sth3<true>(ce, S, s, z);
+        }
+    }
+}
+
+// the site-local updates of step it alone: U' = M(E') U, phi' = phi + (tau +
+// dtau/2) dtau pi' and the traceless part taken by E'.  xb, xa: the states
+// before and after the step; c: a full cotangent set, in place
+__global__ __launch_bounds__(IPG_BLOCK) void k_adj_local(const EvDesc* __restrict__ evs, const double* __restrict__ xb,
+                                                        const double* __restrict__ xa, int it, double* c) {
+    const EvDesc& ev = evs[0];
+    const long long s = xcd_site();
+    if (s >= ev.S) return;
+    const size_t S = ev.S;
     const double dt = ev.dtau, tau = it * dt, g = ev.g;
     const Slot B = slot_of(xb, S), A = slot_of(xa, S);
     const double kappa = g * g * dt / (tau + dt / 2.);
-    {
-        M3 e1b = ldh<true>(pin + kPE1 * S, S, s), ub = m_zero();
-        u_adj(ldm<true>(B.Ux, S, s), ldh<true>(A.E1, S, s), kappa, cin_ux(pin, S, N, i, j, s), ub, e1b);
-        stm<true>(pout + kPU1 * S, S, s, ub);
-        sth<true>(pout + kPE1 * S, S, s, traceless(hproj(e1b)));
-    }
-    {
-        M3 e2b = ldh<true>(pin + kPE2 * S, S, s), ub = m_zero();
-        u_adj(ldm<true>(B.Uy, S, s), ldh<true>(A.E2, S, s), kappa, cin_uy(pin, S, N, i, j, s), ub, e2b);
-        stm<true>(pout + kPU2 * S, S, s, ub);
-        sth<true>(pout + kPE2 * S, S, s, traceless(hproj(e2b)));
-    }
-    const M3 phb = cin_ph(pin, S, N, i, j, s);
-    sth<true>(pout + kPPh * S, S, s, phb);
-    sth<true>(pout + kPPi * S, S, s, ldh<true>(pin + kPPi * S, S, s) + ((tau + dt / 2.) * dt) * phb);
+    H3 z;
+    M3 ub = adj_link_update(ldm<true>(B.Ux, S, s), ldh3<true>(A.E1, S, s), kappa, ldm<true>(c + kPU1 * S, S, s),
+                            ldh3<true>(c + kPE1 * S, S, s), z);
+    stm<true>(c + kPU1 * S, S, s, ub);
+    sth3<true>(c + kPE1 * S, S, s, z);
+    ub = adj_link_update(ldm<true>(B.Uy, S, s), ldh3<true>(A.E2, S, s), kappa, ldm<true>(c + kPU2 * S, S, s),
+                         ldh3<true>(c + kPE2 * S, S, s), z);
+    stm<true>(c + kPU2 * S, S, s, ub);
+    sth3<true>(c + kPE2 * S, S, s, z);
+    sth3<true>(c + kPPi * S, S, s,
+               ldh3<true>(c + kPPi * S, S, s) + ((tau + dt / 2.) * dt) * ldh3<true>(c + kPPh * S, S, s));
 }
 
-// pass 2: the plaquettes of E' (U12 = ux uy_px ux_py^+ uy^+,
-// U1m2 = ux uy_pxmy^+ ux_my^+ uy_my, U2m1 = uy ux_mxpy^+ uy_mx^+ ux_mx)
-__device__ __forceinline__ void adj_plaq_site(const EvDesc& ev, long long s, const double* __restrict__ xb, int it,
-                                              double* __restrict__ pout) {
-    const Lat L{ev.N, ev.S};
-    const size_t S = L.S;
-    const int N = L.N, i = (int)(s / N), j = (int)(s - (long long)i * N);
-    const double dt = ev.dtau, tau = it * dt, g = ev.g;
-    const Slot B = slot_of(xb, S);
-    M3 U12b, U1m2b, U2m1b;
-    plaq_bars(ldh<true>(pout + kPE1 * S, S, s), ldh<true>(pout + kPE2 * S, S, s), tau, dt, g, U12b, U1m2b, U2m1b);
-    M3 B1, B2, B3, B4, uxs, uys;
-    {
-        const M3 ux = ldm<true>(B.Ux, S, s);
-        adj_prod4(ux, ldm<true>(B.Uy, S, L.at(i + 1, j)), dag(ldm<true>(B.Ux, S, L.at(i, j + 1))), dag(ldm<true>(B.Uy, S, s)), U12b,
-                  B1, B2, B3, B4);
-        uxs = B1;
-        stm<true>(pout + (kPOy + 0) * S, S, s, B2);
-        stm<true>(pout + (kPOx + 0) * S, S, s, dag(B3));
-        uys = dag(B4);
-        adj_prod4(ux, dag(ldm<true>(B.Uy, S, L.at(i + 1, j - 1))), dag(ldm<true>(B.Ux, S, L.at(i, j - 1))),
-                  ldm<true>(B.Uy, S, L.at(i, j - 1)), U1m2b, B1, B2, B3, B4);
-    }
-    uxs = uxs + B1;
-    stm<true>(pout + (kPOy + 18) * S, S, s, dag(B2));
-    stm<true>(pout + (kPOx + 18) * S, S, s, dag(B3));
-    stm<true>(pout + (kPOy + 36) * S, S, s, B4);
-    adj_prod4(ldm<true>(B.Uy, S, s), dag(ldm<true>(B.Ux, S, L.at(i - 1, j + 1))), dag(ldm<true>(B.Uy, S, L.at(i - 1, j))),
-              ldm<true>(B.Ux, S, L.at(i - 1, j)), U2m1b, B1, B2, B3, B4);
-    uys = uys + B1;
-    stm<true>(pout + (kPOx + 36) * S, S, s, dag(B2));
-    stm<true>(pout + (kPOy + 54) * S, S, s, dag(B3));
-    stm<true>(pout + (kPOx + 54) * S, S, s, B4);
-    add_m3(pout + kPU1 * S, S, s, uxs);
-    add_m3(pout + kPU2 * S, S, s, uys);
-}
-
-// pass 3: the commutators of E' and the pi' stencil
-//   pi' = pi + (dtau/tau) [Ux phi(x+x) Ux^+ + Ux(x-x)^+ phi(x-x) Ux(x-x) + (y) - 4 phi]
-__device__ __forceinline__ void adj_phi_site(const EvDesc& ev, long long s, const double* __restrict__ xb, int it,
-                                             double* __restrict__ pout) {
-    const Lat L{ev.N, ev.S};
-    const size_t S = L.S;
-    const int N = L.N, i = (int)(s / N), j = (int)(s - (long long)i * N);
-    const double dt = ev.dtau, tau = it * dt;
-    const Slot B = slot_of(xb, S);
-    const cd c2c{0., -dt / tau};  // conj(i dtau / tau)
-    const M3 Bb = (dt / tau) * ldh<true>(pout + kPPi * S, S, s);
-    const M3 ph = ldh<true>(B.phi, S, s);
-    M3 phs = -4. * Bb;
-    {
-        const M3 u = ldm<true>(B.Ux, S, s), pn = ldh<true>(B.phi, S, L.at(i + 1, j));
-        M3 ub = m_zero(), pnb = m_zero();
-        comm_adj(u, pn, ph, cscale(c2c, ldh<true>(pout + kPE1 * S, S, s)), phs, ub, pnb);
-        adj_conj(u, pn, Bb, ub, pnb);
-        add_m3(pout + kPU1 * S, S, s, ub);
-        sth<true>(pout + (kPOph + 0) * S, S, s, hproj(pnb));
-    }
-    {
-        const M3 u = ldm<true>(B.Uy, S, s), pn = ldh<true>(B.phi, S, L.at(i, j + 1));
-        M3 ub = m_zero(), pnb = m_zero();
-        comm_adj(u, pn, ph, cscale(c2c, ldh<true>(pout + kPE2 * S, S, s)), phs, ub, pnb);
-        adj_conj(u, pn, Bb, ub, pnb);
-        add_m3(pout + kPU2 * S, S, s, ub);
-        sth<true>(pout + (kPOph + 9) * S, S, s, hproj(pnb));
-    }
-    {
-        const size_t sm = L.at(i - 1, j);
-        M3 ub = m_zero(), pnb = m_zero();
-        adj_conjd(ldm<true>(B.Ux, S, sm), ldh<true>(B.phi, S, sm), Bb, ub, pnb);
-        add_m3(pout + (kPOx + 54) * S, S, s, ub);
-        sth<true>(pout + (kPOph + 18) * S, S, s, hproj(pnb));
-    }
-    {
-        const size_t sm = L.at(i, j - 1);
-        M3 ub = m_zero(), pnb = m_zero();
-        adj_conjd(ldm<true>(B.Uy, S, sm), ldh<true>(B.phi, S, sm), Bb, ub, pnb);
-        add_m3(pout + (kPOy + 36) * S, S, s, ub);
-        sth<true>(pout + (kPOph + 27) * S, S, s, hproj(pnb));
-    }
-    add_h(pout + kPPh * S, S, s, hproj(phs));
-}
-
-// The three passes as kernels of their own (few matrices live at a time).
-// Each pass reads only its own site's planes of pout, so a site can also run
-// them back to back (below).
-__global__ __launch_bounds__(IPG_BLOCK) void k_adj_local(const EvDesc* __restrict__ evs, const double* __restrict__ xb,
-                                                        const double* __restrict__ xa, int it,
-                                                        const double* __restrict__ pin, double* __restrict__ pout) {
-    const long long s = xcd_site();
-    if (s < evs[0].S) adj_local_site(evs[0], s, xb, xa, it, pin, pout);
-}
-__global__ __launch_bounds__(IPG_BLOCK) void k_adj_plaq(const EvDesc* __restrict__ evs, const double* __restrict__ xb,
-                                                       int it, double* __restrict__ pout) {
-    const long long s = xcd_site();
-    if (s < evs[0].S) adj_plaq_site(evs[0], s, xb, it, pout);
-}
-__global__ __launch_bounds__(IPG_BLOCK) void k_adj_phi(const EvDesc* __restrict__ evs, const double* __restrict__ xb,
-                                                      int it, double* __restrict__ pout) {
-    const long long s = xcd_site();
-    if (s < evs[0].S) adj_phi_site(evs[0], s, xb, it, pout);
-}
-
-
-// The passes back to back with their partial sums on chip: the link
-// cotangents of the own site (pass 1 starts them, passes 2 and 3 add) and the
-// two link outboxes that passes 2 and 3 both write (U_x to (-1,0), U_y to
-// (0,-1)) live in LDS, 72 doubles per thread, until their last term; every
-// other plane of pout is written once, when final.  Kept in pout instead,
-// each of those planes crosses HBM three times (written, read back after the
-// L2 has evicted it, written again).  Same sums in the same order as the
-// three kernels.
-constexpr int kAccSlots = 72;  // U_x, U_y, outbox U_y (0,-1), outbox U_x (-1,0)
-__device__ __forceinline__ M3 acc_ld(const double* a) {
-    M3 m;
-#pragma unroll
-    for (int k = 0; k < 9; k++) {
-        m.e[k].r = a[(2 * k) * IPG_BLOCK];
-        m.e[k].i = a[(2 * k + 1) * IPG_BLOCK];
-    }
-    return m;
-}
-__device__ __forceinline__ void acc_st(double* a, const M3& m) {
-#pragma unroll
-    for (int k = 0; k < 9; k++) {
-        a[(2 * k) * IPG_BLOCK] = m.e[k].r;
-        a[(2 * k + 1) * IPG_BLOCK] = m.e[k].i;
-    }
-}
-// passes 2 and 3 of one site with the partial sums in LDS; the link
-// cotangents of pass 1 come from LDS (P1_LDS) or from pout
-template <bool P1_LDS>
-__device__ __forceinline__ void adj_plaq_phi_lds(const EvDesc& ev, long long s, const double* __restrict__ xb, int it,
-                                                 double* __restrict__ pout, double* aU1) {
-    double* const aU2 = aU1 + 18 * IPG_BLOCK;
-    double* const aOy36 = aU1 + 36 * IPG_BLOCK;
-    double* const aOx54 = aU1 + 54 * IPG_BLOCK;
-    const Lat L{ev.N, ev.S};
-    const size_t S = L.S;
-    const int N = L.N, i = (int)(s / N), j = (int)(s - (long long)i * N);
-    const double dt = ev.dtau, tau = it * dt, g = ev.g;
-    const Slot B = slot_of(xb, S);
-    // pass 2: the plaquettes of E'
-    {
-        M3 U12b, U1m2b, U2m1b;
-        plaq_bars(ldh<true>(pout + kPE1 * S, S, s), ldh<true>(pout + kPE2 * S, S, s), tau, dt, g, U12b, U1m2b, U2m1b);
-        M3 B1, B2, B3, B4, uxs, uys;
-        {
-            const M3 ux = ldm<true>(B.Ux, S, s);
-            adj_prod4(ux, ldm<true>(B.Uy, S, L.at(i + 1, j)), dag(ldm<true>(B.Ux, S, L.at(i, j + 1))), dag(ldm<true>(B.Uy, S, s)),
-                      U12b, B1, B2, B3, B4);
-            uxs = B1;
-            stm<true>(pout + (kPOy + 0) * S, S, s, B2);
-            stm<true>(pout + (kPOx + 0) * S, S, s, dag(B3));
-            uys = dag(B4);
-            adj_prod4(ux, dag(ldm<true>(B.Uy, S, L.at(i + 1, j - 1))), dag(ldm<true>(B.Ux, S, L.at(i, j - 1))),
-                      ldm<true>(B.Uy, S, L.at(i, j - 1)), U1m2b, B1, B2, B3, B4);
-        }
-        uxs = uxs + B1;
-        stm<true>(pout + (kPOy + 18) * S, S, s, dag(B2));
-        stm<true>(pout + (kPOx + 18) * S, S, s, dag(B3));
-        acc_st(aOy36, B4);
-        adj_prod4(ldm<true>(B.Uy, S, s), dag(ldm<true>(B.Ux, S, L.at(i - 1, j + 1))), dag(ldm<true>(B.Uy, S, L.at(i - 1, j))),
-                  ldm<true>(B.Ux, S, L.at(i - 1, j)), U2m1b, B1, B2, B3, B4);
-        uys = uys + B1;
-        stm<true>(pout + (kPOx + 36) * S, S, s, dag(B2));
-        stm<true>(pout + (kPOy + 54) * S, S, s, dag(B3));
-        acc_st(aOx54, B4);
-        acc_st(aU1, (P1_LDS ? acc_ld(aU1) : ldm<true>(pout + kPU1 * S, S, s)) + uxs);
-        acc_st(aU2, (P1_LDS ? acc_ld(aU2) : ldm<true>(pout + kPU2 * S, S, s)) + uys);
-    }
-    asm volatile("" ::: "memory");
-    // pass 3: the commutators of E' and the pi' stencil
-    {
-        const cd c2c{0., -dt / tau};  // conj(i dtau / tau)
-        const M3 Bb = (dt / tau) * ldh<true>(pout + kPPi * S, S, s);
-        const M3 ph = ldh<true>(B.phi, S, s);
-        M3 phs = -4. * Bb;
-        {
-            const M3 u = ldm<true>(B.Ux, S, s), pn = ldh<true>(B.phi, S, L.at(i + 1, j));
-            M3 ub = m_zero(), pnb = m_zero();
-            comm_adj(u, pn, ph, cscale(c2c, ldh<true>(pout + kPE1 * S, S, s)), phs, ub, pnb);
-            adj_conj(u, pn, Bb, ub, pnb);
-            stm<true>(pout + kPU1 * S, S, s, acc_ld(aU1) + ub);
-            sth<true>(pout + (kPOph + 0) * S, S, s, hproj(pnb));
-        }
-        {
-            const M3 u = ldm<true>(B.Uy, S, s), pn = ldh<true>(B.phi, S, L.at(i, j + 1));
-            M3 ub = m_zero(), pnb = m_zero();
-            comm_adj(u, pn, ph, cscale(c2c, ldh<true>(pout + kPE2 * S, S, s)), phs, ub, pnb);
-            adj_conj(u, pn, Bb, ub, pnb);
-            stm<true>(pout + kPU2 * S, S, s, acc_ld(aU2) + ub);
-            sth<true>(pout + (kPOph + 9) * S, S, s, hproj(pnb));
-        }
-        {
-            const size_t sm = L.at(i - 1, j);
-            M3 ub = m_zero(), pnb = m_zero();
-            adj_conjd(ldm<true>(B.Ux, S, sm), ldh<true>(B.phi, S, sm), Bb, ub, pnb);
-            stm<true>(pout + (kPOx + 54) * S, S, s, acc_ld(aOx54) + ub);
-            sth<true>(pout + (kPOph + 18) * S, S, s, hproj(pnb));
-        }
-        {
-            const size_t sm = L.at(i, j - 1);
-            M3 ub = m_zero(), pnb = m_zero();
-            adj_conjd(ldm<true>(B.Uy, S, sm), ldh<true>(B.phi, S, sm), Bb, ub, pnb);
-            stm<true>(pout + (kPOy + 36) * S, S, s, acc_ld(aOy36) + ub);
-            sth<true>(pout + (kPOph + 27) * S, S, s, hproj(pnb));
-        }
-        add_h(pout + kPPh * S, S, s, hproj(phs));
-    }
-}
-__global__ __launch_bounds__(IPG_BLOCK, 1) void k_adj_step_lds(const EvDesc* __restrict__ evs,
-                                                              const double* __restrict__ xb,
-                                                              const double* __restrict__ xa, int it,
-                                                              const double* __restrict__ pin,
-                                                              double* __restrict__ pout) {
-    __shared__ double acc[kAccSlots * IPG_BLOCK];
-    double* const aU1 = acc + threadIdx.x;
-    double* const aU2 = aU1 + 18 * IPG_BLOCK;
-    const EvDesc& ev = evs[0];
-    const Lat L{ev.N, ev.S};
-    const long long s = xcd_site();
-    if (s >= L.S) return;
-    const size_t S = L.S;
-    const int N = L.N, i = (int)(s / N), j = (int)(s - (long long)i * N);
-    const double dt = ev.dtau, tau = it * dt, g = ev.g;
-    const Slot B = slot_of(xb, S), A = slot_of(xa, S);
-    // pass 1: the link update, the traceless part of E', phi' and pi'
-    {
-        const double kappa = g * g * dt / (tau + dt / 2.);
-        {
-            M3 e1b = ldh<true>(pin + kPE1 * S, S, s), ub = m_zero();
-            u_adj(ldm<true>(B.Ux, S, s), ldh<true>(A.E1, S, s), kappa, cin_ux(pin, S, N, i, j, s), ub, e1b);
-            acc_st(aU1, ub);
-            sth<true>(pout + kPE1 * S, S, s, traceless(hproj(e1b)));
-        }
-        {
-            M3 e2b = ldh<true>(pin + kPE2 * S, S, s), ub = m_zero();
-            u_adj(ldm<true>(B.Uy, S, s), ldh<true>(A.E2, S, s), kappa, cin_uy(pin, S, N, i, j, s), ub, e2b);
-            acc_st(aU2, ub);
-            sth<true>(pout + kPE2 * S, S, s, traceless(hproj(e2b)));
-        }
-        const M3 phb = cin_ph(pin, S, N, i, j, s);
-        sth<true>(pout + kPPh * S, S, s, phb);
-        sth<true>(pout + kPPi * S, S, s, ldh<true>(pin + kPPi * S, S, s) + ((tau + dt / 2.) * dt) * phb);
-    }
-    // the partial sums are read back from LDS, not kept in registers
-    asm volatile("" ::: "memory");
-    adj_plaq_phi_lds<true>(ev, s, xb, it, pout, aU1);
-}
-// passes 2 and 3 as one kernel after k_adj_local (the whole-step kernel
-// above spills: pass 1's link exponential reverse and pass 3 do not fit the
-// register file together)
-__global__ __launch_bounds__(IPG_BLOCK, 1) void k_adj_plaq_phi(const EvDesc* __restrict__ evs,
-                                                              const double* __restrict__ xb, int it,
-                                                              double* __restrict__ pout) {
-    __shared__ double acc[kAccSlots * IPG_BLOCK];
-    const long long s = xcd_site();
-    if (s < evs[0].S) adj_plaq_phi_lds<false>(evs[0], s, xb, it, pout, acc + threadIdx.x);
-}
 // ---- the tau = 0 kick (phi += dtau^2/2 pi, U = M(E) U) in reverse ----------------
-// pin: pending cotangents after the kick; cout: compact cotangents of the
+// pin: the cotangent set after the kick; cout: compact cotangents of the
 // tau = 0 fields
 __global__ __launch_bounds__(IPG_BLOCK) void k_adj_kick(const EvDesc* __restrict__ evs, const double* __restrict__ x0,
                                                        const double* __restrict__ pin, double* __restrict__ cout) {
@@ -875,23 +752,22 @@ __global__ __launch_bounds__(IPG_BLOCK) void k_adj_kick(const EvDesc* __restrict
     const long long s = xcd_site();
     if (s >= ev.S) return;
     const size_t S = ev.S;
-    const int N = ev.N, i = (int)(s / N), j = (int)(s - (long long)i * N);
     const double dt = ev.dtau, tau = 0., g = ev.g;
     const Slot X = slot_of(x0, S);
     const double kappa = g * g * dt / (tau + dt / 2.);
     {
         M3 e1b = ldh<true>(pin + kPE1 * S, S, s), ub = m_zero();
-        u_adj(ldm<true>(X.Ux, S, s), ldh<true>(X.E1, S, s), kappa, cin_ux(pin, S, N, i, j, s), ub, e1b);
+        u_adj(ldm<true>(X.Ux, S, s), ldh<true>(X.E1, S, s), kappa, ldm<true>(pin + kPU1 * S, S, s), ub, e1b);
         stm<true>(cot(cout, S, 0), S, s, ub);
         stm<true>(cot(cout, S, 2), S, s, hproj(e1b));
     }
     {
         M3 e2b = ldh<true>(pin + kPE2 * S, S, s), ub = m_zero();
-        u_adj(ldm<true>(X.Uy, S, s), ldh<true>(X.E2, S, s), kappa, cin_uy(pin, S, N, i, j, s), ub, e2b);
+        u_adj(ldm<true>(X.Uy, S, s), ldh<true>(X.E2, S, s), kappa, ldm<true>(pin + kPU2 * S, S, s), ub, e2b);
         stm<true>(cot(cout, S, 1), S, s, ub);
         stm<true>(cot(cout, S, 3), S, s, hproj(e2b));
     }
-    const M3 phb = cin_ph(pin, S, N, i, j, s);
+    const M3 phb = ldh<true>(pin + kPPh * S, S, s);
     stm<true>(cot(cout, S, 4), S, s, phb);
     stm<true>(cot(cout, S, 5), S, s, ldh<true>(pin + kPPi * S, S, s) + ((tau + dt / 2.) * dt) * phb);
 }
@@ -1014,19 +890,17 @@ void ipg_adj_zero(double* p, long long n, hipStream_t st) {
 void ipg_adj_loss(const EvDesc* d, long long S, const double* xs, int it, double yb, double* cout, hipStream_t st) {
     hipLaunchKernelGGL(k_adj_loss, dim3(nb8_of(S)), dim3(IPG_BLOCK), 0, st, d, xs, it, yb, cout);
 }
-void ipg_adj_step(const EvDesc* d, long long S, const double* xb, const double* xa, int it, const double* cin,
-                  double* cout, hipStream_t st, int variant) {
-    if (variant == 1) {
-        hipLaunchKernelGGL(k_adj_step_lds, dim3(nb8_of(S)), dim3(IPG_BLOCK), 0, st, d, xb, xa, it, cin, cout);
-        return;
-    }
-    hipLaunchKernelGGL(k_adj_local, dim3(nb8_of(S)), dim3(IPG_BLOCK), 0, st, d, xb, xa, it, cin, cout);
-    if (variant == 2) {
-        hipLaunchKernelGGL(k_adj_plaq_phi, dim3(nb8_of(S)), dim3(IPG_BLOCK), 0, st, d, xb, it, cout);
-        return;
-    }
-    hipLaunchKernelGGL(k_adj_plaq, dim3(nb8_of(S)), dim3(IPG_BLOCK), 0, st, d, xb, it, cout);
-    hipLaunchKernelGGL(k_adj_phi, dim3(nb8_of(S)), dim3(IPG_BLOCK), 0, st, d, xb, it, cout);
+void ipg_adj_local(const EvDesc* d, long long S, const double* xb, const double* xa, int it, double* c,
+                   hipStream_t st) {
+    hipLaunchKernelGGL(k_adj_local, dim3(nb8_of(S)), dim3(IPG_BLOCK), 0, st, d, xb, xa, it, c);
+}
+void ipg_adj_gather(const EvDesc* d, long long S, const double* xb, const double* xp, int it, const double* cin,
+                    double* cout, hipStream_t st) {
+    const dim3 g(nb8_of(S) * (IPG_BLOCK / kRoleSites)), b(4 * kRoleSites);
+    if (xp)
+        hipLaunchKernelGGL(k_adj_gather<true>, g, b, 0, st, d, xb, xp, it, cin, cout);
+    else
+        hipLaunchKernelGGL(k_adj_gather<false>, g, b, 0, st, d, xb, xb, it, cin, cout);
 }
 void ipg_adj_kick(const EvDesc* d, long long S, const double* x0, const double* cin, double* cout, hipStream_t st) {
     hipLaunchKernelGGL(k_adj_kick, dim3(nb8_of(S)), dim3(IPG_BLOCK), 0, st, d, x0, cin, cout);

@@ -50,14 +50,47 @@ IPG_HD M3 m_one() {
     m.e[0].r = m.e[4].r = m.e[8].r = 1.;
     return m;
 }
+// c + a b, c + a conj(b), c + conj(a) b and c - a b.  Written as a + b * c
+// on whole complex numbers a product takes a multiply, a multiply-add and an
+// add per component; as a chain of multiply-adds it takes two instructions.
+// (The host builds, which only check the algebra, take the plain expression.)
+IPG_HD double ipg_fma(double a, double b, double c) {
+#ifdef __HIP_DEVICE_COMPILE__
+    return __builtin_fma(a, b, c);
+#else
+    return a * b + c;
+#endif
+}
+IPG_HD cd cfma(cd a, cd b, cd c) {
+    return cd{ipg_fma(-a.i, b.i, ipg_fma(a.r, b.r, c.r)), ipg_fma(a.i, b.r, ipg_fma(a.r, b.i, c.i))};
+}
+IPG_HD cd cfma_bc(cd a, cd b, cd c) {
+    return cd{ipg_fma(a.i, b.i, ipg_fma(a.r, b.r, c.r)), ipg_fma(-a.r, b.i, ipg_fma(a.i, b.r, c.i))};
+}
+IPG_HD cd cfma_ac(cd a, cd b, cd c) {
+    return cd{ipg_fma(a.i, b.i, ipg_fma(a.r, b.r, c.r)), ipg_fma(-a.i, b.r, ipg_fma(a.r, b.i, c.i))};
+}
+IPG_HD cd cfma(cd a, double s, cd c) { return cd{ipg_fma(a.r, s, c.r), ipg_fma(a.i, s, c.i)}; }
 IPG_HD M3 operator*(const M3& a, const M3& b) {
     M3 c;
 #pragma unroll
     for (int i = 0; i < 3; i++)
 #pragma unroll
         for (int j = 0; j < 3; j++)
-            c.e[3 * i + j] = a.e[3 * i] * b.e[j] + a.e[3 * i + 1] * b.e[3 + j] + a.e[3 * i + 2] * b.e[6 + j];
+            c.e[3 * i + j] =
+                cfma(a.e[3 * i + 2], b.e[6 + j], cfma(a.e[3 * i + 1], b.e[3 + j], a.e[3 * i] * b.e[j]));
     return c;
+}
+// c + a * b
+IPG_HD M3 mac(const M3& c, const M3& a, const M3& b) {
+    M3 r;
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+#pragma unroll
+        for (int j = 0; j < 3; j++)
+            r.e[3 * i + j] = cfma(a.e[3 * i + 2], b.e[6 + j],
+                                  cfma(a.e[3 * i + 1], b.e[3 + j], cfma(a.e[3 * i], b.e[j], c.e[3 * i + j])));
+    return r;
 }
 // a * b^dagger
 IPG_HD M3 mul_bd(const M3& a, const M3& b) {
@@ -66,8 +99,8 @@ IPG_HD M3 mul_bd(const M3& a, const M3& b) {
     for (int i = 0; i < 3; i++)
 #pragma unroll
         for (int j = 0; j < 3; j++)
-            c.e[3 * i + j] = mulc(a.e[3 * i], b.e[3 * j]) + mulc(a.e[3 * i + 1], b.e[3 * j + 1]) +
-                             mulc(a.e[3 * i + 2], b.e[3 * j + 2]);
+            c.e[3 * i + j] = cfma_bc(a.e[3 * i + 2], b.e[3 * j + 2],
+                                     cfma_bc(a.e[3 * i + 1], b.e[3 * j + 1], mulc(a.e[3 * i], b.e[3 * j])));
     return c;
 }
 // a^dagger * b
@@ -77,8 +110,19 @@ IPG_HD M3 mul_ad(const M3& a, const M3& b) {
     for (int i = 0; i < 3; i++)
 #pragma unroll
         for (int j = 0; j < 3; j++)
-            c.e[3 * i + j] = cmul(a.e[i], b.e[j]) + cmul(a.e[3 + i], b.e[3 + j]) + cmul(a.e[6 + i], b.e[6 + j]);
+            c.e[3 * i + j] = cfma_ac(a.e[6 + i], b.e[6 + j], cfma_ac(a.e[3 + i], b.e[3 + j], cmul(a.e[i], b.e[j])));
     return c;
+}
+// c + a^dagger * b
+IPG_HD M3 mac_ad(const M3& c, const M3& a, const M3& b) {
+    M3 r;
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+#pragma unroll
+        for (int j = 0; j < 3; j++)
+            r.e[3 * i + j] = cfma_ac(a.e[6 + i], b.e[6 + j],
+                                     cfma_ac(a.e[3 + i], b.e[3 + j], cfma_ac(a.e[i], b.e[j], c.e[3 * i + j])));
+    return r;
 }
 IPG_HD M3 dag(const M3& a) {
     M3 c;
@@ -285,6 +329,15 @@ IPG_HD H3 operator+(const H3& a, const H3& b) {
     }
     return c;
 }
+IPG_HD H3 operator-(const H3& a, const H3& b) {
+    H3 c;
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        c.d[k] = a.d[k] - b.d[k];
+        c.o[k] = a.o[k] - b.o[k];
+    }
+    return c;
+}
 IPG_HD H3 operator*(double s, const H3& a) {
     H3 c;
 #pragma unroll
@@ -307,8 +360,8 @@ IPG_HD M3 mul_hd(const H3& h, const M3& u) {
 #pragma unroll
         for (int j = 0; j < 3; j++) {
             const int k = (i + 1) % 3, l = (i + 2) % 3;
-            c.e[3 * i + j] =
-                (cconj(u.e[3 * j + i]) * h.d[i] + mulc(h_off(h, i, k), u.e[3 * j + k])) + mulc(h_off(h, i, l), u.e[3 * j + l]);
+            c.e[3 * i + j] = cfma_bc(h_off(h, i, l), u.e[3 * j + l],
+                                     cfma_bc(h_off(h, i, k), u.e[3 * j + k], cconj(u.e[3 * j + i]) * h.d[i]));
         }
     return c;
 }
@@ -320,9 +373,34 @@ IPG_HD M3 mul_h(const H3& h, const M3& u) {
 #pragma unroll
         for (int j = 0; j < 3; j++) {
             const int k = (i + 1) % 3, l = (i + 2) % 3;
-            c.e[3 * i + j] = (u.e[3 * i + j] * h.d[i] + h_off(h, i, k) * u.e[3 * k + j]) + h_off(h, i, l) * u.e[3 * l + j];
+            c.e[3 * i + j] = cfma(h_off(h, i, l), u.e[3 * l + j], cfma(h_off(h, i, k), u.e[3 * k + j], u.e[3 * i + j] * h.d[i]));
         }
     return c;
+}
+// U H
+IPG_HD M3 mul_mh(const M3& u, const H3& h) {
+    M3 c;
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+#pragma unroll
+        for (int j = 0; j < 3; j++) {
+            const int k = (j + 1) % 3, l = (j + 2) % 3;
+            c.e[3 * i + j] = cfma(u.e[3 * i + l], h_off(h, l, j), cfma(u.e[3 * i + k], h_off(h, k, j), u.e[3 * i + j] * h.d[j]));
+        }
+    return c;
+}
+// c + U H
+IPG_HD M3 mac_mh(const M3& c, const M3& u, const H3& h) {
+    M3 r;
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+#pragma unroll
+        for (int j = 0; j < 3; j++) {
+            const int k = (j + 1) % 3, l = (j + 2) % 3;
+            r.e[3 * i + j] = cfma(u.e[3 * i + l], h_off(h, l, j),
+                                  cfma(u.e[3 * i + k], h_off(h, k, j), cfma(u.e[3 * i + j], h.d[j], c.e[3 * i + j])));
+        }
+    return r;
 }
 // the product A B where it is Hermitian
 IPG_HD H3 herm_mul(const M3& a, const M3& b) {
@@ -331,13 +409,14 @@ IPG_HD H3 herm_mul(const M3& a, const M3& b) {
     for (int i = 0; i < 3; i++) {
         double t = 0.;
 #pragma unroll
-        for (int k = 0; k < 3; k++) t += a.e[3 * i + k].r * b.e[3 * k + i].r - a.e[3 * i + k].i * b.e[3 * k + i].i;
+        for (int k = 0; k < 3; k++)
+            t = ipg_fma(-a.e[3 * i + k].i, b.e[3 * k + i].i, ipg_fma(a.e[3 * i + k].r, b.e[3 * k + i].r, t));
         h.d[i] = t;
     }
 #pragma unroll
     for (int q = 0; q < 3; q++) {
         const int i = q == 2 ? 1 : 0, j = q == 0 ? 1 : 2;
-        h.o[q] = a.e[3 * i] * b.e[j] + a.e[3 * i + 1] * b.e[3 + j] + a.e[3 * i + 2] * b.e[6 + j];
+        h.o[q] = cfma(a.e[3 * i + 2], b.e[6 + j], cfma(a.e[3 * i + 1], b.e[3 + j], a.e[3 * i] * b.e[j]));
     }
     return h;
 }
@@ -348,13 +427,14 @@ IPG_HD H3 herm_mul_ad(const M3& a, const M3& b) {
     for (int i = 0; i < 3; i++) {
         double t = 0.;
 #pragma unroll
-        for (int k = 0; k < 3; k++) t += a.e[3 * k + i].r * b.e[3 * k + i].r + a.e[3 * k + i].i * b.e[3 * k + i].i;
+        for (int k = 0; k < 3; k++)
+            t = ipg_fma(a.e[3 * k + i].i, b.e[3 * k + i].i, ipg_fma(a.e[3 * k + i].r, b.e[3 * k + i].r, t));
         h.d[i] = t;
     }
 #pragma unroll
     for (int q = 0; q < 3; q++) {
         const int i = q == 2 ? 1 : 0, j = q == 0 ? 1 : 2;
-        h.o[q] = cmul(a.e[i], b.e[j]) + cmul(a.e[3 + i], b.e[3 + j]) + cmul(a.e[6 + i], b.e[6 + j]);
+        h.o[q] = cfma_ac(a.e[6 + i], b.e[6 + j], cfma_ac(a.e[3 + i], b.e[3 + j], cmul(a.e[i], b.e[j])));
     }
     return h;
 }
@@ -371,15 +451,16 @@ IPG_HD AH ah_mul(const M3& a, const M3& b) {
     for (int i = 0; i < 3; i++) {
         double t = 0.;
 #pragma unroll
-        for (int k = 0; k < 3; k++) t += a.e[3 * i + k].r * b.e[3 * k + i].i + a.e[3 * i + k].i * b.e[3 * k + i].r;
+        for (int k = 0; k < 3; k++)
+            t = ipg_fma(a.e[3 * i + k].i, b.e[3 * k + i].r, ipg_fma(a.e[3 * i + k].r, b.e[3 * k + i].i, t));
         h.d[i] = 2. * t;
     }
 #pragma unroll
     for (int q = 0; q < 3; q++) {
         const int i = q == 2 ? 1 : 0, j = q == 0 ? 1 : 2;
-        const cd up = a.e[3 * i] * b.e[j] + a.e[3 * i + 1] * b.e[3 + j] + a.e[3 * i + 2] * b.e[6 + j];
-        const cd lo = a.e[3 * j] * b.e[i] + a.e[3 * j + 1] * b.e[3 + i] + a.e[3 * j + 2] * b.e[6 + i];
-        h.o[q] = up - cconj(lo);
+        cd lo = cfma(a.e[3 * j + 2], b.e[6 + i], cfma(a.e[3 * j + 1], b.e[3 + i], a.e[3 * j] * b.e[i]));
+        lo = cd{-lo.r, lo.i};
+        h.o[q] = cfma(a.e[3 * i + 2], b.e[6 + j], cfma(a.e[3 * i + 1], b.e[3 + j], cfma(a.e[3 * i], b.e[j], lo)));
     }
     return h;
 }
@@ -425,6 +506,59 @@ IPG_HD AH operator-(const AH& a, const AH& b) {
         c.o[k] = a.o[k] - b.o[k];
     }
     return c;
+}
+// -i k A of an anti-Hermitian matrix: Hermitian
+IPG_HD H3 herm_mi(double k, const AH& a) {
+    H3 h;
+#pragma unroll
+    for (int q = 0; q < 3; q++) {
+        h.d[q] = k * a.d[q];
+        h.o[q] = cd{k * a.o[q].i, -k * a.o[q].r};
+    }
+    return h;
+}
+// s e + e s of two Hermitian matrices
+IPG_HD H3 anticommutator(const H3& s, const H3& e) {
+    H3 h;
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+        const int k = (i + 1) % 3, l = (i + 2) % 3;
+        const cd sk = h_off(s, i, k), ek = h_off(e, i, k), sl = h_off(s, i, l), el = h_off(e, i, l);
+        h.d[i] = 2. * (s.d[i] * e.d[i] + (sk.r * ek.r + sk.i * ek.i) + (sl.r * el.r + sl.i * el.i));
+    }
+#pragma unroll
+    for (int q = 0; q < 3; q++) {
+        const int i = q == 2 ? 1 : 0, j = q == 0 ? 1 : 2, m = 3 - i - j;
+        h.o[q] = (e.o[q] * (s.d[i] + s.d[j]) + s.o[q] * (e.d[i] + e.d[j])) +
+                 (h_off(s, i, m) * h_off(e, m, j) + h_off(e, i, m) * h_off(s, m, j));
+    }
+    return h;
+}
+IPG_HD H3 h_traceless(H3 a) {
+    const double t = (a.d[0] + a.d[1] + a.d[2]) / 3.0;
+    a.d[0] -= t;
+    a.d[1] -= t;
+    a.d[2] -= t;
+    return a;
+}
+// A - A^+ and A + A^+
+IPG_HD AH ah_of(const M3& a) {
+    AH h;
+#pragma unroll
+    for (int i = 0; i < 3; i++) h.d[i] = 2. * a.e[4 * i].i;
+    h.o[0] = a.e[1] - cconj(a.e[3]);
+    h.o[1] = a.e[2] - cconj(a.e[6]);
+    h.o[2] = a.e[5] - cconj(a.e[7]);
+    return h;
+}
+IPG_HD H3 two_herm(const M3& a) {
+    H3 h;
+#pragma unroll
+    for (int i = 0; i < 3; i++) h.d[i] = 2. * a.e[4 * i].r;
+    h.o[0] = a.e[1] + cconj(a.e[3]);
+    h.o[1] = a.e[2] + cconj(a.e[6]);
+    h.o[2] = a.e[5] + cconj(a.e[7]);
+    return h;
 }
 // (1 + X + X^2/2) with X = i c E, E Hermitian: X^2 = -c^2 E^2
 IPG_HD M3 taylor2(double c, const H3& e) {
