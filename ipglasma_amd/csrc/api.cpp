@@ -338,7 +338,7 @@ struct Engine {
     double* d_Q = nullptr;
     bool have_table = false;
     int* d_flag = nullptr;
-    int* d_work = nullptr;    // root-finder work counter
+    int* d_work = nullptr;    // root-finder work counter and list lengths
     double* d_out = nullptr;  // 16 doubles per event (8 results + scratch)
     double* d_obs = nullptr;  // kObs doubles per event (Landau, eccentricities)
     int nblk = 0, nlinkblk = 0;
@@ -568,7 +568,7 @@ struct Engine {
         nlinkblk = lb0;
         HIPCHK(hipMalloc(&d_desc, sizeof(EvDesc) * nev));
         HIPCHK(hipMalloc(&d_flag, sizeof(int) * nev));
-        HIPCHK(hipMalloc(&d_work, sizeof(int)));
+        HIPCHK(hipMalloc(&d_work, sizeof(int) * (nev + 1)));
         HIPCHK(hipMalloc(&d_out, sizeof(double) * 16 * nev));
         HIPCHK(hipMalloc(&d_obs, sizeof(double) * kObs * nev));
         HIPCHK(hipMemset(d_obs, 0, sizeof(double) * kObs * nev));
@@ -894,21 +894,7 @@ struct Engine {
     int fields() {
         const int nev = (int)ev.size();
         ipg_launch_links(d_desc, nev, nblk, st);
-        {
-            int maxN = 0;
-            for (const EvDesc& d : desc)
-                if (d.active) maxN = std::max(maxN, d.N);
-            int nact = 0;
-            for (const EvDesc& d : desc) nact += d.active;
-            const std::string key =
-                "newton_waves_per_simd/N=" + std::to_string(maxN) + "/events=" + std::to_string(nact);
-            bool meas = false;
-            const int v = g_tuner.pick(key, 3, &meas);
-            hipEvent_t a, b;
-            if (timed_begin(key, v, meas, &a, &b)) (void)hipEventRecord(a, st);
-            ipg_launch_newton(d_desc, nev, nlinkblk, d_work, v + 1, st);
-            if (b) (void)hipEventRecord(b, st);
-        }
+        ipg_launch_newton(d_desc, nev, nlinkblk, d_work, st);
         ipg_launch_newton_stats(d_desc, nev, nlinkblk, d_out, st);
         ipg_launch_pi_init(d_desc, nev, nblk, st);
         ipg_launch_zero_fields(d_desc, nev, nblk, st);

@@ -11,6 +11,8 @@
 //                 (Init.cpp:2459-2491)
 //   k_newton      per-link root finder (Init.cpp:3344-3481)
 //   k_pi_init     pi = -(2i/g) A^eta (Init.cpp:2521-2584, 2664-2680)
+#include <algorithm>
+
 #include "ipg_device.hpp"
 #include "ipg_internal.hpp"
 #include "fft_lds.hpp"
@@ -871,37 +873,275 @@ __device__ __forceinline__ void restart_alpha(uint64_t seed, uint32_t link, uint
     normals8(seed, draw, 0xFFFF0000u, link, al);
 }
 
-// F_a = -Im[tr t^a (W - W^+) + tr t^a (W U^+ - U W^+)]
-__device__ __forceinline__ double residual(const M3& W, const M3& Us, const cd trc[8], double F[8]) {
-    M3 Mt = mul_bd(W, Us) - mul_bd(Us, W);
-    cd t[8];
-    tr_gen(Mt, t);
+// F_a = -Im[tr t^a (W - W^+) + tr t^a (W U^+ - U W^+)]; trci[a] is the first
+// trace.  The second matrix is W U^+ minus its own conjugate, so one product
+// gives both; returns sum |F_a|
+__device__ __forceinline__ double residual(const M3& W, const M3& Us, const double (&trci)[8], double (&F)[8]) {
+    const AH m = ah_of(mul_bd(W, Us));
+    const double s3 = 1.0 / (2.0 * sqrt(3.0));
+    const double t[8] = {m.o[0].i, m.o[0].r, 0.5 * (m.d[0] - m.d[1]), m.o[1].i, m.o[1].r, m.o[2].i, m.o[2].r,
+                         s3 * (m.d[0] + m.d[1]) - 2.0 * s3 * m.d[2]};
     double Fz = 0.;
 #pragma unroll
     for (int a = 0; a < 8; a++) {
-        F[a] = -(trc[a].i + t[a].i);
+        F[a] = -(trci[a] + t[a]);
         Fz += fabs(F[a]);
     }
     return Fz;
 }
-
-// Root finder, one link per group of NG = 8 lanes (Init.cpp:3386-3476).
-// Lane c of a group evaluates Jacobian column c (one SU(3) exponential) and
-// owns row c of the 8x9 augmented system during the pivoted elimination, so
-// an iteration costs one exponential of latency instead of nine.  Every lane
-// of a group carries the same link state and computes the residual, the
-// update and the next iterate redundantly; the per-element arithmetic (and
-// its order) is that of the serial algorithm.  A group takes its next link
-// from a wave-aggregated work counter as soon as its link is done.
-constexpr int NG = 8;
-
-__device__ __forceinline__ double pick8(const double (&v)[8], int c) {
-    double r = v[0];
+// the finite-difference steps and the exponent of Jacobian column c: the
+// serial loop adds the step to alpha[b] and subtracts it again in place, so
+// column c sees (alpha[k] + d_k) - d_k for k < c; returns d_c
+__device__ __forceinline__ double column_exponent(const double (&alpha)[8], int c, double (&p)[8]) {
+    double d = 0.;
 #pragma unroll
-    for (int k = 1; k < 8; k++)
-        if (k == c) r = v[k];
-    return r;
+    for (int k = 0; k < 8; k++) {
+        const double dk = fmax(0.001, fmin(10., 0.01 * fabs(alpha[k])));
+        p[k] = k < c ? (alpha[k] + dk) - dk : (k == c ? alpha[k] + dk : alpha[k]);
+        if (k == c) d = dk;
+    }
+    return d;
 }
+// the column 2 Im tr t^a W D / d, D = (E - Us)^+; false where the reference's running
+// sum |J_a| stays below 1e-15 (it then takes the analytic Jacobian)
+__device__ __forceinline__ bool jacobian_column(const M3& W, const M3& D, double d, double (&col)[8]) {
+    const M3 Mp = W * D;
+    cd t[8];
+    tr_gen(Mp, t);
+    double chk = 0.;
+    bool good = true;
+#pragma unroll
+    for (int a = 0; a < 8; a++) {
+        col[a] = 2. * t[a].i / d;
+        chk += fabs(col[a]);
+        if (chk < 1e-15) good = false;
+    }
+    return good;
+}
+// the analytic column about U = Us
+__device__ __forceinline__ void analytic_column(const M3& W, const M3& Us, int c, double (&col)[8]) {
+    const M3 Mb = gen_mul(c, dag(Us));
+#pragma unroll
+    for (int a = 0; a < 8; a++) col[a] = -2. * retrprod(gen_mul(a, W), Mb);
+}
+// J y = F by Gaussian elimination with partial pivoting (first maximal pivot),
+// J row-major, in registers; y replaces F.  Rows are exchanged by selects, and
+// only when some lane of the wavefront has an exchange to make.
+__device__ __forceinline__ void solve_rows(double (&J)[64], double (&F)[8]) {
+#pragma unroll
+    for (int j = 0; j < 7; j++) {
+        double best = fabs(J[9 * j]);
+        int p = j;
+#pragma unroll
+        for (int r = j + 1; r < 8; r++)
+            if (fabs(J[8 * r + j]) > best) {
+                best = fabs(J[8 * r + j]);
+                p = r;
+            }
+        if (__any(p != j)) {
+#pragma unroll
+            for (int r = j + 1; r < 8; r++) {
+                const bool sw = r == p;
+#pragma unroll
+                for (int c = j; c < 8; c++) {
+                    const double x = J[8 * j + c], y = J[8 * r + c];
+                    J[8 * j + c] = sw ? y : x;
+                    J[8 * r + c] = sw ? x : y;
+                }
+                const double x = F[j], y = F[r];
+                F[j] = sw ? y : x;
+                F[r] = sw ? x : y;
+            }
+        }
+        const double inv = J[9 * j] != 0. ? 1. / J[9 * j] : 0.;
+#pragma unroll
+        for (int r = j + 1; r < 8; r++) {
+            const double f = J[8 * r + j] * inv;
+#pragma unroll
+            for (int c = j + 1; c < 8; c++) J[8 * r + c] -= f * J[8 * j + c];
+            F[r] -= f * F[j];
+        }
+    }
+#pragma unroll
+    for (int r = 7; r >= 0; r--) {
+        double t = F[r];
+#pragma unroll
+        for (int c = r + 1; c < 8; c++) t -= J[8 * r + c] * F[c];
+        F[r] = t / J[9 * r];
+    }
+}
+
+// First pass of the root finder: four lanes per link, 16 links a wavefront.
+// Each lane evaluates two Jacobian columns; the system goes through LDS and
+// every lane solves it in registers.  The first iteration starts from exponent
+// 0 at every link, so its column exponentials are the same everywhere and come
+// from a table.  Almost every link converges in two to six iterations (mean
+// 2.1 to 4.0 over the lattices in use); one that has not after kQuadIter, that
+// wants a restart, or that polishes goes to its event's list for k_newton,
+// which starts it afresh.
+// FP64 issue bounds it, most of it in the exponentials.  N = 512 (2.1
+// iterations a link) / N = 128 (3.2): eight lanes a link, all of them repeating
+// the residual, the update and its exponential, with the elimination by
+// shuffles 1740 / 380 us; this 1020 + 244 / 98 + 9 us (both passes).  Two lanes a link with the columns in
+// registers is less work, but spills at two waves per SIMD (1324 / 190 us).
+constexpr int kQuadIter = 8;
+constexpr int kQuadLinks = 16;
+__global__ __launch_bounds__(64, 2) void k_newton_quad(const EvDesc* __restrict__ evs, int nev, int* __restrict__ cnt) {
+    __shared__ double mU0[18][kQuadLinks], mW[18][kQuadLinks], mUs[18][kQuadLinks];
+    __shared__ double mJ[64][kQuadLinks];  // row-major
+    __shared__ double tab[8][18];          // exp(i d t^c), d the first step
+    const int lane = threadIdx.x;
+    const int sub = lane & 3, k = lane >> 2;
+    constexpr int kPer = NWB / kQuadLinks;  // blocks per 64-link block
+    const int e = find_event_links(evs, nev, (int)blockIdx.x / kPer);
+    const EvDesc& ev = evs[e];
+    if (!ev.active) return;
+    const long long S = ev.S;
+    const long long l = ((long long)blockIdx.x - (long long)kPer * ev.lblock0) * kQuadLinks + k;
+    // 2 S is a multiple of 512: a block is full or past the end
+    if (l - k >= 2 * S) return;
+    const int dir = l >= S;
+    const long long s = dir ? l - S : l;
+    const bool direct = ev.newton_polish == 0;
+    auto ld = [&](const double (*m)[kQuadLinks]) {
+        // read where used: kept in registers across the loops they spill
+        asm volatile("" ::: "memory");
+        M3 r;
+#pragma unroll
+        for (int q = 0; q < 9; q++) r.e[q] = cd{m[2 * q][k], m[2 * q + 1][k]};
+        return r;
+    };
+    auto st = [&](double (*m)[kQuadLinks], const M3& r) {
+#pragma unroll
+        for (int q = 0; q < 9; q++) {
+            m[2 * q][k] = r.e[q].r;
+            m[2 * q + 1][k] = r.e[q].i;
+        }
+    };
+    double alpha[8];
+#pragma unroll
+    for (int a = 0; a < 8; a++) alpha[a] = 0.;
+    if (direct) {
+        if (lane < 8) {
+            double p[8];
+            (void)column_exponent(alpha, lane, p);
+            const M3 E = exp_iQt(p);
+#pragma unroll
+            for (int q = 0; q < 9; q++) {
+                tab[lane][2 * q] = E.e[q].r;
+                tab[lane][2 * q + 1] = E.e[q].i;
+            }
+        }
+        const M3 U1 = ldm(dir ? ev.L1y : ev.L1x, S, s);
+        const M3 U2 = ldm(dir ? ev.L2y : ev.L2x, S, s);
+        if (sub == 0) {
+            const M3 U0 = U1 * U2;
+            st(mU0, U0);
+            st(mW, U1 + U2);
+            // exp(0) is the identity (its closed form gives no number, the guard 1)
+            st(mUs, U0);
+        }
+    }
+    bool done = !direct, failed = !direct;
+    int analytic = 0;
+    __syncthreads();
+    for (int iter = 1; iter <= kQuadIter && __any(!done); iter++) {
+        // not unrolled: one copy of the exponential keeps the kernel inside the
+        // instruction cache
+        bool good = true;
+#pragma unroll 1
+        for (int q = 0; q < 2; q++) {
+            const int c = 2 * sub + q;
+            double p[8], col[8];
+            const double d = column_exponent(alpha, c, p);
+            M3 E;
+            if (iter == 1) {
+#pragma unroll
+                for (int r = 0; r < 9; r++) E.e[r] = cd{tab[c][2 * r], tab[c][2 * r + 1]};
+            } else {
+                E = exp_iQt(p);
+            }
+            E = E * ld(mU0);
+            E = dag(E) - dag(ld(mUs));
+            good = jacobian_column(ld(mW), E, d, col) && good;
+#pragma unroll
+            for (int a = 0; a < 8; a++) mJ[8 * a + c][k] = col[a];
+        }
+        const unsigned long long bad = __ballot(!good);
+        if ((bad >> (lane & ~3)) & 15ull) {
+            analytic = 1;
+#pragma unroll 1
+            for (int q = 0; q < 2; q++) {
+                double col[8];
+                analytic_column(ld(mW), ld(mUs), 2 * sub + q, col);
+#pragma unroll
+                for (int a = 0; a < 8; a++) mJ[8 * a + 2 * sub + q][k] = col[a];
+            }
+        }
+        double F[8];
+        double Fzero;
+        {
+            const M3 W = ld(mW);
+            cd trc[8];
+            tr_gen(W - dag(W), trc);
+            double trci[8];
+#pragma unroll
+            for (int a = 0; a < 8; a++) trci[a] = trc[a].i;
+            Fzero = residual(W, ld(mUs), trci, F);
+        }
+        __syncthreads();
+        {
+            double J[64];
+#pragma unroll
+            for (int a = 0; a < 64; a++) J[a] = mJ[a][k];
+            solve_rows(J, F);
+        }
+        bool okstep = true;
+#pragma unroll
+        for (int a = 0; a < 8; a++) {
+            if (fabs(F[a]) > 1e5) okstep = false;
+            const double dk = fmax(0.001, fmin(10., 0.01 * fabs(alpha[a])));
+            alpha[a] = ((alpha[a] + dk) - dk) + F[a];
+        }
+        M3 Us = exp_iQt(alpha);
+        Us = Us * ld(mU0);
+        __syncthreads();
+        if (sub == 0 && !done) st(mUs, Us);
+        if (!done) {
+            if (!okstep) {
+                done = failed = true;
+            } else if (!(Fzero > 1e-6)) {
+                done = true;
+                if (sub == 0) {
+                    stm(ev.U[0][dir], S, s, Us);
+                    ev.newton_stat[l] = iter | (analytic << 29);
+                }
+            }
+        }
+        __syncthreads();
+    }
+    if (!done) failed = true;
+    // unfinished links, one entry each
+    const unsigned long long m = __ballot(failed && sub == 0);
+    if (m) {
+        const int first = __ffsll((long long)m) - 1;
+        int base = 0;
+        if (lane == first) base = atomicAdd(&cnt[1 + e], __popcll(m));
+        base = __shfl(base, first, 64);
+        if (failed && sub == 0)
+            ((int*)ev.land_epsv)[base + __popcll(m & ((1ull << lane) - 1ull))] = (int)l;
+    }
+}
+
+// The links k_newton_quad leaves, one per group of NG = 8 lanes
+// (Init.cpp:3386-3476): a few links in a million take tens to thousands of
+// iterations, so here the latency of an iteration counts.  Lane c of a group
+// evaluates Jacobian column c (one SU(3) exponential); every lane carries the
+// same link state and computes the residual, the elimination (in registers:
+// through shuffles it was a third of the iteration), the update and the next
+// iterate redundantly.  A group takes its next link from a wave-aggregated
+// work counter as soon as its link is done.
+constexpr int NG = 8;
 
 __device__ __forceinline__ M3 lds_m3(const double* p) {
     M3 m;
@@ -917,9 +1157,17 @@ __device__ __forceinline__ void lds_st(double* p, const M3& m) {
     }
 }
 
-template <int OCC>
-__global__ __launch_bounds__(NWB, OCC) void k_newton(const EvDesc* __restrict__ evs, int nev, int nitems,
-                                                     int* __restrict__ counter) {
+// exp(i best t) U0, or the identity, into out; out of line: 200 restarts without
+// a root are rare
+__device__ __attribute__((noinline)) void best_iterate(const double* best, const double* U0, int one, double* out) {
+    double ba[8];
+#pragma unroll
+    for (int a = 0; a < 8; a++) ba[a] = best[a];
+    lds_st(out, one ? m_one() : exp_iQt(ba) * lds_m3(U0));
+}
+
+// cnt[0]: the work counter, cnt[1 + e]: the length of event e's list
+__global__ __launch_bounds__(NWB, 1) void k_newton(const EvDesc* __restrict__ evs, int nev, int* __restrict__ cnt) {
     __shared__ double Jt[NWB / NG][8][8];  // [group][row a][column c]
     // per group: U0 = U1 U2, W = U1 + U2, the iterate Us (written by lane 0)
     __shared__ double Ms[NWB / NG][3][18];
@@ -957,19 +1205,22 @@ __global__ __launch_bounds__(NWB, OCC) void k_newton(const EvDesc* __restrict__ 
         if (need) {
             const int first = __ffsll((long long)need) - 1;
             int base = 0;
-            if (lane == first) base = atomicAdd(counter, __popcll(need));
+            if (lane == first) base = atomicAdd(cnt, __popcll(need));
             base = __shfl(base, first, NWB);
             int g = lead_need ? base + __popcll(need & ((1ull << lane) - 1ull)) : 0;
             g = __shfl(g, 0, NG);
             if (state == 0) {
-                if (g >= nitems) {
+                // entry g of the events' lists, one after the other
+                e = 0;
+                while (e < nev && g >= cnt[1 + e]) g -= cnt[1 + e++];
+                if (e >= nev) {
                     state = 2;
+                    e = 0;
                 } else {
-                    e = find_event_links(evs, nev, g / NWB);
                     const EvDesc& ev = evs[e];
-                    l = (long long)g - (long long)ev.lblock0 * NWB;
                     const long long S = ev.S;
-                    if (ev.active && l < 2 * S) {
+                    l = ((const int*)ev.land_epsv)[g];
+                    {
                         dir = l >= S;
                         s = dir ? l - S : l;
                         link = (uint32_t)(2 * s + dir);
@@ -986,7 +1237,8 @@ __global__ __launch_bounds__(NWB, OCC) void k_newton(const EvDesc* __restrict__ 
                             for (int a = 0; a < 8; a++) trci[a] = trc[a].i;
                             lds_st(mU0, U0);
                             lds_st(mW, W);
-                            lds_st(mUs, exp_iQt(alpha) * U0);
+                            // exp(0) is the identity (its closed form gives no number, the guard 1)
+                            lds_st(mUs, U0);
                         }
                         best_one = 1;
                         Fzero = 10.;
@@ -995,7 +1247,6 @@ __global__ __launch_bounds__(NWB, OCC) void k_newton(const EvDesc* __restrict__ 
                         ndraw = 0;
                         state = 1;
                     }
-                    // padding slot or inactive event: ask again
                 }
             }
         }
@@ -1008,44 +1259,22 @@ __global__ __launch_bounds__(NWB, OCC) void k_newton(const EvDesc* __restrict__ 
         total++;
         double F[8];
         {
-            const M3 W = lds_m3(mW), Us = lds_m3(mUs);
-            M3 Mt = mul_bd(W, Us) - mul_bd(Us, W);
-            cd t[8];
-            tr_gen(Mt, t);
-            Fzero = 0.;
+            double tr8[8];
 #pragma unroll
-            for (int a = 0; a < 8; a++) {
-                F[a] = -(trci[a] + t[a].i);
-                Fzero += fabs(F[a]);
-            }
+            for (int a = 0; a < 8; a++) tr8[a] = trci[a];
+            Fzero = residual(lds_m3(mW), lds_m3(mUs), tr8, F);
         }
         double col[8];
         bool good = true;
         if (npol == 0) {
-            // the serial loop adds the step to alpha[b] and subtracts it again
-            // in place, so column b sees (alpha[k] + d_k) - d_k for k < b
-            double dk[8], ar[8], p[8];
+            double p[8];
+            const double d = column_exponent(alpha, c, p);
+            good = jacobian_column(lds_m3(mW), dag(exp_iQt(p) * lds_m3(mU0)) - dag(lds_m3(mUs)), d, col);
 #pragma unroll
             for (int k = 0; k < 8; k++) {
-                dk[k] = fmax(0.001, fmin(10., 0.01 * fabs(alpha[k])));
-                ar[k] = (alpha[k] + dk[k]) - dk[k];
+                const double dk = fmax(0.001, fmin(10., 0.01 * fabs(alpha[k])));
+                alpha[k] = (alpha[k] + dk) - dk;
             }
-#pragma unroll
-            for (int k = 0; k < 8; k++) p[k] = k < c ? ar[k] : (k == c ? alpha[k] + dk[k] : alpha[k]);
-            const double d = pick8(dk, c);
-            const M3 E = exp_iQt(p) * lds_m3(mU0);
-            M3 Mp = lds_m3(mW) * (dag(E) - dag(lds_m3(mUs)));
-            cd t[8];
-            tr_gen(Mp, t);
-            double chk = 0.;
-#pragma unroll
-            for (int a = 0; a < 8; a++) {
-                col[a] = 2. * t[a].i / d;
-                chk += fabs(col[a]);
-                if (chk < 1e-15) good = false;
-            }
-#pragma unroll
-            for (int k = 0; k < 8; k++) alpha[k] = ar[k];
         } else {
             // newton_polish: the exact Jacobian about the iterate,
             // U <- exp(i beta^a t^a) U, J_ab = -2 Re tr(t^a W U^+ t^b)
@@ -1058,100 +1287,49 @@ __global__ __launch_bounds__(NWB, OCC) void k_newton(const EvDesc* __restrict__ 
         const unsigned long long bad = __ballot(!good);
         if (npol == 0 && ((bad >> (grp * NG)) & 0xFFull)) {
             analytic = 1;
-            const M3 Mb = gen_mul(c, dag(lds_m3(mUs)));
-            const M3 W = lds_m3(mW);
-#pragma unroll
-            for (int a = 0; a < 8; a++) col[a] = -2. * retrprod(gen_mul(a, W), Mb);
+            analytic_column(lds_m3(mW), lds_m3(mUs), c, col);
         }
-        // ---- columns -> rows
+        // ---- the columns of the group's lanes
 #pragma unroll
         for (int a = 0; a < 8; a++) Jt[grp][a][c] = col[a];
         __syncthreads();
-        double row[9];
+        double J[64];
 #pragma unroll
-        for (int k = 0; k < 8; k++) row[k] = Jt[grp][c][k];
-        row[8] = pick8(F, c);
+        for (int k = 0; k < 64; k++) J[k] = Jt[grp][k >> 3][k & 7];
         __syncthreads();
-        // ---- Gaussian elimination with partial pivoting (first maximal
-        // pivot); row swaps carry the right-hand side along
-#pragma unroll
-        for (int j = 0; j < 7; j++) {
-            double key = c >= j ? fabs(row[j]) : -1.;
-            int idx = c >= j ? c : NG;
-#pragma unroll
-            for (int m = 1; m < NG; m <<= 1) {
-                const double ok = __shfl_xor(key, m, NG);
-                const int oi = __shfl_xor(idx, m, NG);
-                if (ok > key || (ok == key && oi < idx)) {
-                    key = ok;
-                    idx = oi;
-                }
-            }
-            // no pivot above |a_jj| keeps row j (NaN entries are never taken)
-            const double ajj0 = __shfl(fabs(row[j]), j, NG);
-            const int ip = (idx < NG && key > ajj0) ? idx : j;
-            const int src = c == j ? ip : (c == ip ? j : c);
-#pragma unroll
-            for (int k = 0; k < 9; k++) row[k] = __shfl(row[k], src, NG);
-            double piv[8];
-#pragma unroll
-            for (int k = j; k < 8; k++) piv[k] = __shfl(row[k], j, NG);
-            const double ajj = piv[j];
-            if (c > j && ajj != 0.0) {
-                const double arj = row[j] / ajj;
-                row[j] = arj;
-#pragma unroll
-                for (int k = j + 1; k < 8; k++) row[k] = row[k] - arj * piv[k];
-            }
-        }
-        // ---- unit-lower forward, upper back substitution on column 8
-#pragma unroll
-        for (int cc = 0; cc < 7; cc++) {
-            const double yc = __shfl(row[8], cc, NG);
-            if (c > cc) row[8] -= row[cc] * yc;
-        }
-        double y[8];
-        if (c == 7) row[8] = row[8] / row[7];
-        y[7] = __shfl(row[8], 7, NG);
-#pragma unroll
-        for (int r = 6; r >= 0; r--) {
-            if (c == r) {
-                double t = row[8];
-#pragma unroll
-                for (int cc = r + 1; cc < 8; cc++) t -= row[cc] * y[cc];
-                row[8] = t / row[r];
-            }
-            y[r] = __shfl(row[8], r, NG);
-        }
+        solve_rows(J, F);
+        double(&y)[8] = F;
         bool okstep = true;
 #pragma unroll
         for (int a = 0; a < 8; a++)
             if (fabs(y[a]) > 1e5) okstep = false;
-        M3 Us;
-        if (npol > 0) {
-            Us = exp_iQt(y) * lds_m3(mUs);
-        } else {
+        if (npol == 0) {
             if (okstep) {
 #pragma unroll
                 for (int a = 0; a < 8; a++) alpha[a] = alpha[a] + y[a];
             } else {
                 restart_alpha(evs[e].newton_seed, link, ndraw++, alpha);
             }
-            Us = exp_iQt(alpha) * lds_m3(mU0);
-        }
-        if (npol == 0 && Fzero < Fmin) {
-            // best = Us, kept as its exponent (Us is exp(i alpha t) U0)
-            Fmin = Fzero;
-            if (c == 0)
+            if (Fzero < Fmin) {
+                // best = the new iterate, kept as its exponent (Us is exp(i alpha t) U0)
+                Fmin = Fzero;
+                if (c == 0)
 #pragma unroll
-                for (int a = 0; a < 8; a++) best_alpha[a] = alpha[a];
-            best_one = 0;
+                    for (int a = 0; a < 8; a++) best_alpha[a] = alpha[a];
+                best_one = 0;
+            }
+            if (iter == maxIt) {
+                restart_alpha(evs[e].newton_seed, link, ndraw++, alpha);
+                nRestart++;
+                iter = 0;
+            }
         }
-        if (npol == 0 && iter == maxIt) {
-            restart_alpha(evs[e].newton_seed, link, ndraw++, alpha);
-            Us = exp_iQt(alpha) * lds_m3(mU0);
-            nRestart++;
-            iter = 0;
+        M3 Us;
+        {
+            double q[8];
+#pragma unroll
+            for (int a = 0; a < 8; a++) q[a] = npol > 0 ? y[a] : alpha[a];
+            Us = exp_iQt(q) * lds_m3(npol > 0 ? mUs : mU0);
         }
         if (c == 0) lds_st(mUs, Us);
         bool stop = state == 1 && !(Fzero > 1e-6 && iter < maxIt && nRestart < maxRe);
@@ -1164,14 +1342,11 @@ __global__ __launch_bounds__(NWB, OCC) void k_newton(const EvDesc* __restrict__ 
             const EvDesc& ev = evs[e];
             const int conv = nRestart != maxRe;
             if (c == 0) {
-                M3 out = Us;
                 if (!conv) {
-                    double ba[8];
-#pragma unroll
-                    for (int a = 0; a < 8; a++) ba[a] = best_alpha[a];
-                    out = best_one ? m_one() : exp_iQt(ba) * lds_m3(mU0);
+                    best_iterate(best_alpha, mU0, best_one, mUs);
+                    Us = lds_m3(mUs);
                 }
-                stm(ev.U[0][dir], ev.S, s, out);
+                stm(ev.U[0][dir], ev.S, s, Us);
                 ev.newton_stat[l] = total | (nRestart << 20) | ((!conv) << 28) | (analytic << 29);
             }
             state = 0;
@@ -1380,24 +1555,17 @@ void ipg_launch_unit_v(const EvDesc* d, int nev, int nblk, hipStream_t st) {
 void ipg_launch_links(const EvDesc* d, int nev, int nblk, hipStream_t st) {
     hipLaunchKernelGGL(k_links, dim3(nblk), dim3(IPG_BLOCK), 0, st, d, nev);
 }
-__global__ void k_zero_counter(int* c) { *c = 0; }
+__global__ void k_zero_counters(int* c, int n) {
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t < n) c[t] = 0;
+}
 
-// variant = waves per SIMD the kernel is compiled for (1, 2, 3: fewer
-// registers, more spill); every variant computes the same result
-void ipg_launch_newton(const EvDesc* d, int nev, int nlinkblk, int* d_counter, int variant, hipStream_t st) {
-    // persistent single-wave blocks, enough to fill the machine at the
-    // variant's occupancy (256 CUs x 4 SIMDs); each loops until the work
-    // counter runs out
-    const int occ = variant < 1 ? 1 : (variant > 3 ? 3 : variant);
-    int grid = 1024 * occ;
-    if (grid > nlinkblk) grid = nlinkblk;
-    hipLaunchKernelGGL(k_zero_counter, dim3(1), dim3(1), 0, st, d_counter);
-    if (occ == 3)
-        hipLaunchKernelGGL(k_newton<3>, dim3(grid), dim3(NWB), 0, st, d, nev, nlinkblk * NWB, d_counter);
-    else if (occ == 2)
-        hipLaunchKernelGGL(k_newton<2>, dim3(grid), dim3(NWB), 0, st, d, nev, nlinkblk * NWB, d_counter);
-    else
-        hipLaunchKernelGGL(k_newton<1>, dim3(grid), dim3(NWB), 0, st, d, nev, nlinkblk * NWB, d_counter);
+// d_cnt: 1 + nev ints.  The second pass is persistent: enough one-wave blocks
+// for a wave on every SIMD (256 CUs x 4); each loops until the lists run out.
+void ipg_launch_newton(const EvDesc* d, int nev, int nlinkblk, int* d_cnt, hipStream_t st) {
+    hipLaunchKernelGGL(k_zero_counters, dim3((unsigned)(nev + 1 + 255) / 256), dim3(256), 0, st, d_cnt, nev + 1);
+    hipLaunchKernelGGL(k_newton_quad, dim3(NWB / kQuadLinks * nlinkblk), dim3(NWB), 0, st, d, nev, d_cnt);
+    hipLaunchKernelGGL(k_newton, dim3(std::min(1024, nlinkblk)), dim3(NWB), 0, st, d, nev, d_cnt);
 }
 
 // per event: sum, max of the link iteration counts, restarts, unconverged
