@@ -79,18 +79,27 @@ struct EvDesc {
     double* obs;        // 32 doubles of end-of-evolution observables
 };
 
-// block -> (event, local block) for site-parallel launches
+// block -> event for site-parallel and link-parallel launches: the last event
+// whose first block is not after b.  The lanes of a wavefront look at 64
+// events at once (a loop over the events is a chain of scalar loads of a
+// cache line each, ~0.2 us an event, at the start of every block); call with
+// all lanes of the wavefront active.
+template <typename First>
+__device__ __forceinline__ int find_event_by(int nev, int b, First first) {
+    if (nev == 1) return 0;
+    const int lane = (int)(threadIdx.x & 63);
+    int n = 0;
+    for (int k0 = 0; k0 < nev; k0 += 64) {
+        const int k = k0 + lane;
+        n += __popcll(__ballot(k < nev && b >= first(k)));
+    }
+    return __builtin_amdgcn_readfirstlane(n - 1);
+}
 __device__ __forceinline__ int find_event(const EvDesc* __restrict__ ev, int nev, int b) {
-    int e = 0;
-    for (int k = 1; k < nev; k++)
-        if (b >= ev[k].block0) e = k;
-    return e;
+    return find_event_by(nev, b, [&](int k) { return ev[k].block0; });
 }
 __device__ __forceinline__ int find_event_links(const EvDesc* __restrict__ ev, int nev, int b) {
-    int e = 0;
-    for (int k = 1; k < nev; k++)
-        if (b >= ev[k].lblock0) e = k;
-    return e;
+    return find_event_by(nev, b, [&](int k) { return ev[k].lblock0; });
 }
 
 // Spread consecutive logical blocks over one XCD: hardware dispatches block b

