@@ -841,8 +841,7 @@ struct Engine {
             for (int e : es) minNy = std::min(minNy, desc[e].Ny);
             auto chunk = [&](const EvDesc* dd, int n, int k0, int kcc, int ny) {
                 // keyed by the launch's own event count and chunk length; the
-                // 512-thread forms of the forward row and column passes are
-                // candidates from N = 512 on
+                // forward row pass has candidates from N = 256 on
                 const std::string tail = "/N=" + std::to_string(kv.first) + "/events=" + std::to_string(n) +
                                          "/kc=" + std::to_string(kcc);
                 SetvVariant v;
@@ -858,6 +857,8 @@ struct Engine {
                     // (forward rows 3: 2 with the twiddles in LDS)
                     v.fwd = g_tuner.pick("setv_rows_fwd_block" + tail, 4, &meas);
                     timed_begin("setv_rows_fwd_block" + tail, v.fwd, meas && full, &t.fwd[0], &t.fwd[1]);
+                }
+                {
                     v.cols = g_tuner.pick("setv_cols_block" + tail, 3, &meas);
                     timed_begin("setv_cols_block" + tail, v.cols, meas && full, &t.cols[0], &t.cols[1]);
                 }

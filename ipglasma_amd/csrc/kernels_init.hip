@@ -504,24 +504,36 @@ __global__ __launch_bounds__(IPG_BLOCK) void k_stats_finish(const EvDesc* __rest
 // rows, synchronising itself only
 // TWL: the twiddle table copied into LDS first (LDS reads in the stages
 // instead of global ones)
-template <int N, int BLK = IPG_BLOCK, bool WAVE = false, bool TWL = false>
+// RPB: lattice rows a block takes (1 with WAVE); below N = 256 several, so that
+// every thread of the block has a site and a butterfly (at N = 128 one row
+// gave 128 of 256 threads a site and 64 a radix-8 butterfly: 18.7 -> 15.9 us a
+// chunk)
+constexpr int setv_rows_per_block(int N) {
+    int r = 1;
+    while (2 * r * N <= 256 && N % (2 * r) == 0) r *= 2;
+    return r;
+}
+template <int N, int BLK = IPG_BLOCK, bool WAVE = false, bool TWL = false, int RPB = 1>
 __global__ __launch_bounds__(BLK) void k_setv_rows_fwd(const EvDesc* __restrict__ evs, FftPlanDev pl, int k0,
                                                       int kc) {
-    __shared__ double2 lds[ipgfft::lds_slots(N, 4)];
+    static_assert(N % RPB == 0 && (!WAVE || RPB == 1), "rows per block");
+    __shared__ double2 lds[ipgfft::lds_slots(N, 4 * RPB)];
     __shared__ double2 tws[TWL ? N : 1];
-    const int per_ev = 2 * kc * N;
+    constexpr int NR = N / RPB;
+    const int per_ev = 2 * kc * NR;
     const int e = blockIdx.x / per_ev;
     const int rem = blockIdx.x - e * per_ev;
-    const int n = rem / (kc * N);
-    const int kk = (rem / N) % kc;
-    const int i = rem % N;
+    const int n = rem / (kc * NR);
+    const int kk = (rem / NR) % kc;
+    const int i = (rem % NR) * RPB;
     const int k = k0 + kk;
     const EvDesc& ev = evs[e];
     if (!ev.active || k >= ev.Ny) return;
     const size_t S = ev.S;
     const double* g2 = n ? ev.g2B : ev.g2A;
-    for (int j = threadIdx.x; j < N; j += blockDim.x) {
-        const size_t s = (size_t)i * N + j;
+    for (int q = threadIdx.x; q < RPB * N; q += BLK) {
+        const int r = RPB == 1 ? 0 : q / N, j = q - r * N;
+        const size_t s = (size_t)i * N + q;
         double z[8];
         if (ev.znorm) {
             const double* zp = ev.znorm + (((size_t)n * ev.Ny + k) * S + s) * 8;
@@ -532,7 +544,8 @@ __global__ __launch_bounds__(BLK) void k_setv_rows_fwd(const EvDesc* __restrict_
         }
         const double amp = ev.g * sqrt(g2[s] / (double)ev.Ny);
 #pragma unroll
-        for (int p = 0; p < 4; p++) lds[ipgfft::at(N, p, j)] = make_double2(amp * z[2 * p], amp * z[2 * p + 1]);
+        for (int p = 0; p < 4; p++)
+            lds[ipgfft::at(N, 4 * r + p, j)] = make_double2(amp * z[2 * p], amp * z[2 * p + 1]);
     }
     const double2* tw = pl.tw;
     if constexpr (TWL) {
@@ -545,12 +558,12 @@ __global__ __launch_bounds__(BLK) void k_setv_rows_fwd(const EvDesc* __restrict_
         ipgfft::wave_fft<N, 1, false>(lds + ipgfft::at(N, (int)(threadIdx.x >> 6), 0), tw);
         __syncthreads();
     } else {
-        ipgfft::lds_fft<N, 4, BLK, false>(lds, tw);
+        ipgfft::lds_fft<N, 4 * RPB, BLK, false>(lds, tw);
     }
-    double2* out = ev.fftbuf + ((size_t)n * kc + kk) * 4 * S;
-    for (int q = threadIdx.x; q < 4 * N; q += blockDim.x) {
-        const int p = q / N, j = q - p * N;
-        out[(size_t)p * S + (size_t)i * N + j] = lds[ipgfft::at(N, p, j)];
+    double2* out = ev.fftbuf + ((size_t)n * kc + kk) * 4 * S + (size_t)i * N;
+    for (int q = threadIdx.x; q < 4 * RPB * N; q += BLK) {
+        const int p = q / (RPB * N), t = q - p * (RPB * N), r = RPB == 1 ? 0 : t / N;
+        out[(size_t)p * S + t] = lds[ipgfft::at(N, 4 * r + p, t - r * N)];
     }
 }
 
@@ -1505,35 +1518,56 @@ void ipg_launch_stats(const EvDesc* d, int nev, int nblk, double* out, hipStream
 // v.inv = 2, 3: the prefetching inverse row pass in 512-thread blocks and
 // in 256-thread blocks with wavefront-synchronised transforms; v.inv = 4, 5
 // and v.fwd = 3: variants 0, 1 and 2 with the twiddles read from LDS (5 held
-// to 128 registers, four waves per SIMD).  Each pass is bracketed by its
+// to 128 registers, four waves per SIMD).  Below N = 256 the forward row pass
+// takes several lattice rows a block (the inverse one, serial in the slices,
+// keeps one: two rows a block left half of the CUs without a block, 28 -> 37
+// us a chunk at N = 128).  Each pass is bracketed by its
 // pair of events when they are given.
+// the column pass in the launch shape of variant cv 
+template <int N>
+static void launch_cols(const EvDesc* d, const FftPlanDev& pl, int k0, int kc, int ncol, int cv, hipStream_t st) {
+    constexpr int C = ipgfft::cols_per_block(N);
+    constexpr int CW = C < 8 ? C : 8;
+    if (cv == 1)
+        hipLaunchKernelGGL((k_setv_cols<N, 512>), dim3(ncol), dim3(512), 0, st, d, pl, k0, kc);
+    else if (cv == 2)
+        hipLaunchKernelGGL((k_setv_cols<N, 64 * CW, true>), dim3(ncol), dim3(64 * CW), 0, st, d, pl, k0, kc);
+    else
+        hipLaunchKernelGGL((k_setv_cols<N, IPG_BLOCK>), dim3(ncol), dim3(IPG_BLOCK), 0, st, d, pl, k0, kc);
+}
+template <int N>
+static void launch_rows_fwd(const EvDesc* d, int nev, const FftPlanDev& pl, int k0, int kc, int v, hipStream_t st) {
+    constexpr int R = setv_rows_per_block(N);
+    const dim3 g((unsigned)(nev * 2 * kc * (N / R)));
+    if constexpr (N >= 256) {
+        if (v == 1) {
+            hipLaunchKernelGGL((k_setv_rows_fwd<N, 512>), g, dim3(512), 0, st, d, pl, k0, kc);
+            return;
+        }
+        if (v == 2) {
+            hipLaunchKernelGGL((k_setv_rows_fwd<N, 256, true>), g, dim3(256), 0, st, d, pl, k0, kc);
+            return;
+        }
+        if (v == 3) {
+            hipLaunchKernelGGL((k_setv_rows_fwd<N, 256, true, true>), g, dim3(256), 0, st, d, pl, k0, kc);
+            return;
+        }
+    }
+    hipLaunchKernelGGL((k_setv_rows_fwd<N, IPG_BLOCK, false, false, R>), g, dim3(IPG_BLOCK), 0, st, d, pl, k0, kc);
+}
 template <int N>
 static void setv_chunk(const EvDesc* d, int nev, const FftPlanDev& pl, int k0, int kc, const SetvVariant& v,
                        const SetvEvents& t, hipStream_t st) {
     constexpr int C = ipgfft::cols_per_block(N);
-    const int nrow_fwd = nev * 2 * kc * N;
     const int ncol = nev * 2 * kc * 4 * (N / C);
     const int nrow_inv = nev * 2 * N;
     const int inv_variant = v.inv;
     const hipEvent_t ev_a = t.inv[0], ev_b = t.inv[1];
-    constexpr int CW = C < 8 ? C : 8;  // wavefronts of the wavefront column pass
     if (t.fwd[0]) (void)hipEventRecord(t.fwd[0], st);
-    if (v.fwd == 1 && N >= 256)
-        hipLaunchKernelGGL((k_setv_rows_fwd<N, 512>), dim3(nrow_fwd), dim3(512), 0, st, d, pl, k0, kc);
-    else if (v.fwd == 2 && N >= 256)
-        hipLaunchKernelGGL((k_setv_rows_fwd<N, 256, true>), dim3(nrow_fwd), dim3(256), 0, st, d, pl, k0, kc);
-    else if (v.fwd == 3 && N >= 256)
-        hipLaunchKernelGGL((k_setv_rows_fwd<N, 256, true, true>), dim3(nrow_fwd), dim3(256), 0, st, d, pl, k0, kc);
-    else
-        hipLaunchKernelGGL((k_setv_rows_fwd<N, IPG_BLOCK>), dim3(nrow_fwd), dim3(IPG_BLOCK), 0, st, d, pl, k0, kc);
+    launch_rows_fwd<N>(d, nev, pl, k0, kc, v.fwd, st);
     if (t.fwd[1]) (void)hipEventRecord(t.fwd[1], st);
     if (t.cols[0]) (void)hipEventRecord(t.cols[0], st);
-    if (v.cols == 1 && N >= 256)
-        hipLaunchKernelGGL((k_setv_cols<N, 512>), dim3(ncol), dim3(512), 0, st, d, pl, k0, kc);
-    else if (v.cols == 2 && N >= 256)
-        hipLaunchKernelGGL((k_setv_cols<N, 64 * CW, true>), dim3(ncol), dim3(64 * CW), 0, st, d, pl, k0, kc);
-    else
-        hipLaunchKernelGGL((k_setv_cols<N, IPG_BLOCK>), dim3(ncol), dim3(IPG_BLOCK), 0, st, d, pl, k0, kc);
+    launch_cols<N>(d, pl, k0, kc, ncol, v.cols, st);
     if (t.cols[1]) (void)hipEventRecord(t.cols[1], st);
     if (ev_a) (void)hipEventRecord(ev_a, st);
     if (inv_variant == 1)
@@ -1571,18 +1605,6 @@ void ipg_launch_setv_chunk(const EvDesc* d, int nev, const FftPlanDev& pl, int k
     }
 #undef IPG_SETV_CASE
 }
-// the column pass in the launch shape of variant cv (as setv_chunk)
-template <int N>
-static void launch_cols(const EvDesc* d, const FftPlanDev& pl, int k0, int kc, int ncol, int cv, hipStream_t st) {
-    constexpr int C = ipgfft::cols_per_block(N);
-    constexpr int CW = C < 8 ? C : 8;
-    if (cv == 1 && N >= 256)
-        hipLaunchKernelGGL((k_setv_cols<N, 512>), dim3(ncol), dim3(512), 0, st, d, pl, k0, kc);
-    else if (cv == 2 && N >= 256)
-        hipLaunchKernelGGL((k_setv_cols<N, 64 * CW, true>), dim3(ncol), dim3(64 * CW), 0, st, d, pl, k0, kc);
-    else
-        hipLaunchKernelGGL((k_setv_cols<N, IPG_BLOCK>), dim3(ncol), dim3(IPG_BLOCK), 0, st, d, pl, k0, kc);
-}
 template <int N>
 static void adj_setv_chunk(const EvDesc* d, const FftPlanDev& pl, int k0, int kc, double* vv, double* vbar,
                            double* grad, const SetvVariant& v, hipStream_t st, bool recompute) {
@@ -1592,14 +1614,7 @@ static void adj_setv_chunk(const EvDesc* d, const FftPlanDev& pl, int k0, int kc
     // recompute the chunk's A_k (forward row and column passes) unless the
     // buffer already holds them
     if (recompute) {
-        if (v.fwd == 1 && N >= 256)
-            hipLaunchKernelGGL((k_setv_rows_fwd<N, 512>), dim3(nrow), dim3(512), 0, st, d, pl, k0, kc);
-        else if (v.fwd == 2 && N >= 256)
-            hipLaunchKernelGGL((k_setv_rows_fwd<N, 256, true>), dim3(nrow), dim3(256), 0, st, d, pl, k0, kc);
-        else if (v.fwd == 3 && N >= 256)
-            hipLaunchKernelGGL((k_setv_rows_fwd<N, 256, true, true>), dim3(nrow), dim3(256), 0, st, d, pl, k0, kc);
-        else
-            hipLaunchKernelGGL((k_setv_rows_fwd<N, IPG_BLOCK>), dim3(nrow), dim3(IPG_BLOCK), 0, st, d, pl, k0, kc);
+        launch_rows_fwd<N>(d, 1, pl, k0, kc, v.fwd, st);
         launch_cols<N>(d, pl, k0, kc, ncol, v.cols, st);
     }
     hipLaunchKernelGGL((k_adj_setv_rows<N, 256>), dim3(2 * N), dim3(256), 0, st, d, pl, k0, kc, vv, vbar);
