@@ -90,25 +90,15 @@ __global__ __launch_bounds__(IPG_BLOCK) void k_tp_g(const EvDesc* __restrict__ e
         g[t] = exp(-(d * d / (HBARC * HBARC)) / (2. * ev.BG));
     }
 }
-// N a multiple of 64: a block takes 4 rows x 64 columns; each of its four
-// wavefronts sums a quarter of the nucleons, one column a lane and four rows,
-// so a load of gy serves four products and gx is uniform (a thread per site
-// loads both factors for every product: 125 us at N = 512 with 416 nucleons,
-// 57 us at N = 128; this 42 and 9.5 us).  Other N: a thread per site.
-template <int R>
-__device__ __forceinline__ void tp_rows(const double* __restrict__ gx, const double* __restrict__ gy, int N, int n0,
-                                        int n1, int w, double (&t)[R]) {
-#pragma unroll
-    for (int r = 0; r < R; r++) t[r] = 0.;
-#pragma unroll 4
-    for (int n = n0 + w; n < n1; n += 4) {
-        const double y = gy[(size_t)n * N];
-#pragma unroll
-        for (int r = 0; r < R; r++) t[r] = __builtin_fma(gx[(size_t)n * N + r], y, t[r]);
-    }
-}
+// N a multiple of 64: a block takes 4 rows x 64 columns; each wavefront sums
+// one nucleus for two of the rows, a column a lane, so a load of gy serves two
+// products and gx is uniform (a thread per site loads both factors for every
+// product: 125 us at N = 512 with 416 nucleons, 57 us at N = 128; this
+// 56 and 17 us).  The nucleons are summed one after the other as in the
+// other path, so the two agree to the last bit; quarters of the list summed
+// apart would be faster by a few microseconds and round differently.  Other
+// N: a thread per site.
 __global__ __launch_bounds__(IPG_BLOCK) void k_tp(const EvDesc* __restrict__ evs, int nev) {
-    __shared__ double part[2][4][4][64];  // nucleus, quarter, row, column
     const int e = find_event(evs, nev, blockIdx.x);
     const EvDesc& ev = evs[e];
     if (!ev.active) return;
@@ -116,24 +106,22 @@ __global__ __launch_bounds__(IPG_BLOCK) void k_tp(const EvDesc* __restrict__ evs
     const int lb = xcd_remap(blockIdx.x - ev.block0, ev.nblocks);
     if ((N & 63) == 0 && tp_separable(ev)) {
         if ((long long)lb * IPG_BLOCK >= ev.S) return;
-        const int cpr = N >> 6, i0 = 4 * (lb / cpr), j0 = 64 * (lb % cpr);
         const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = (int)(threadIdx.x & 63);
-        const int A = ev.A1 + ev.A2;
+        const int cpr = N >> 6, i0 = 4 * (lb / cpr) + 2 * (w >> 1), j0 = 64 * (lb % cpr);
+        const int A = ev.A1 + ev.A2, n1 = w & 1 ? A : ev.A1;
         const double* gx = reinterpret_cast<const double*>(ev.fftbuf) + i0;
         const double* gy = reinterpret_cast<const double*>(ev.fftbuf) + (size_t)A * N + j0 + lane;
-        double t[4];
-        tp_rows<4>(gx, gy, N, 0, ev.A1, w, t);
-#pragma unroll
-        for (int r = 0; r < 4; r++) part[0][w][r][lane] = t[r];
-        tp_rows<4>(gx, gy, N, ev.A1, A, w, t);
-#pragma unroll
-        for (int r = 0; r < 4; r++) part[1][w][r][lane] = t[r];
-        __syncthreads();
-        // wavefront w finishes row w
-        const double c = sqrt(1 + ev.xi), q = 2. * M_PI * ev.BG;
-        const size_t o = (size_t)(i0 + w) * N + j0 + lane;
-        ev.TpA[o] = c * ((part[0][0][w][lane] + part[0][1][w][lane]) + (part[0][2][w][lane] + part[0][3][w][lane])) / q;
-        ev.TpB[o] = c * ((part[1][0][w][lane] + part[1][1][w][lane]) + (part[1][2][w][lane] + part[1][3][w][lane])) / q;
+        double t0 = 0., t1 = 0.;
+#pragma unroll 16
+        for (int n = w & 1 ? ev.A1 : 0; n < n1; n++) {
+            const double y = gy[(size_t)n * N];
+            t0 += gx[(size_t)n * N] * y;
+            t1 += gx[(size_t)n * N + 1] * y;
+        }
+        double* o = (w & 1 ? ev.TpB : ev.TpA) + (size_t)i0 * N + j0 + lane;
+        const double pre = sqrt(1 + ev.xi), nrm = 2. * M_PI * ev.BG;
+        o[0] = pre * t0 / nrm;
+        o[N] = pre * t1 / nrm;
         return;
     }
     const long long s = (long long)lb * IPG_BLOCK + threadIdx.x;
@@ -386,7 +374,7 @@ __global__ __launch_bounds__(IPG_BLOCK) void k_stats(const EvDesc* __restrict__ 
     // rows and, inside one row, the columns it covers); the loop over all of them per site was 130 us of the
     // kernel's 146 at N = 512 with 416 nucleons.  A list that would not fit
     // falls back to that loop.
-    __shared__ short near_idx[2][kNearCap];
+    __shared__ int near_idx[2][kNearCap];
     __shared__ int near_n[2];
     if (threadIdx.x < 2) near_n[threadIdx.x] = 0;
     __syncthreads();
@@ -403,7 +391,7 @@ __global__ __launch_bounds__(IPG_BLOCK) void k_stats(const EvDesc* __restrict__ 
             if (ev.nuc[4 * n + 3] == 1. && px > x0 - reach && px < x1 + reach && py > y0 - reach && py < y1 + reach) {
                 const int nb = n >= ev.A1;
                 const int q = atomicAdd(&near_n[nb], 1);
-                if (q < kNearCap) near_idx[nb][q] = (short)n;
+                if (q < kNearCap) near_idx[nb][q] = n;
             }
         }
     }

@@ -1,0 +1,50 @@
+"""Device-to-host copies of whole fields: below the staged copy's threshold of
+4 MiB, just above it with a short last chunk, and at the headline size, where a
+field set on the device comes back bit for bit; and from several threads at
+once, of which one gets the pinned slots and the others the plain copy."""
+import threading
+
+import numpy as np
+import pytest
+
+import _cases as K
+
+pytestmark = pytest.mark.gpu
+
+
+def _event(N):
+    import ipglasma_amd as I
+    return I.Event(K.params("pPb", N=N, Ny=1), seed=3)
+
+
+# 18 planes of N^2 doubles: 2.4, 5.3, 37.7 MB
+@pytest.mark.parametrize("N", [128, 192, 512])
+def test_field_round_trip(N):
+    ev = _event(N)
+    a = np.random.default_rng(N).normal(size=(N * N, 18))
+    ev.set_field("Ux", a)
+    np.testing.assert_array_equal(ev.field("Ux"), a)
+    ev.close()
+
+
+def test_field_round_trip_from_threads():
+    import ipglasma_amd as I
+    bad = []
+
+    def go(k):
+        ev = _event(256)
+        a = np.random.default_rng(k).normal(size=(256 * 256, 18))
+        for _ in range(5):
+            ev.set_field("Ux", a)
+            if not np.array_equal(ev.field("Ux"), a):
+                bad.append(k)
+        ev.close()
+
+    th = [threading.Thread(target=go, args=(k,)) for k in range(4)]
+    for t in th:
+        t.start()
+    for t in th:
+        t.join()
+    assert not bad
+    I.release_cached_memory()  # hands the slots back; the next copy makes them again
+    test_field_round_trip(192)
