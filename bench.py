@@ -495,7 +495,7 @@ def main():
         return
     seeds = list(range(1000, 1000 + a.batch))
     # untimed runs until the autotuner has decided every launch variant of
-    # this workload (evolution schedule, root-finder occupancy, inverse-row
+    # this workload (evolution schedule, site order of the step, inverse-row
     # block): each variant is timed three times on the real workload first
     tune_runs = 0
     while tune_runs < 12:

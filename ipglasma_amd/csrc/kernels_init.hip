@@ -9,7 +9,7 @@
 //                 inverse FFT, V <- exp(-i A.t) V  (Init.cpp:1678-1850)
 //   k_links       U^(1,2)_{x,y} = V(x) V(x+i)^+ with the NaN guard
 //                 (Init.cpp:2459-2491)
-//   k_newton      per-link root finder (Init.cpp:3344-3481)
+//   k_newton_quad, k_newton  per-link root finder (Init.cpp:3344-3481)
 //   k_pi_init     pi = -(2i/g) A^eta (Init.cpp:2521-2584, 2664-2680)
 #include <algorithm>
 
