@@ -33,6 +33,7 @@
 #include <thread>
 #include <vector>
 
+#include "copy_out.hpp"
 #include "host.hpp"
 #include "ipg_internal.hpp"
 #include "fft_lds.hpp"
@@ -248,92 +249,6 @@ void block_release(void* p, size_t n) {
         }
     }
     (void)hipFree(p);
-}
-// Device-to-host copies of fields and gradients.  A copy into pageable memory
-// goes through the runtime's staging buffer on one thread, which also takes
-// the page faults of a fresh destination (4 GB/s measured, 17 GB/s once the
-// pages are there, against 56 GB/s into pinned memory).  Large copies go
-// through kCopyThreads pinned slots instead, each with a thread and a stream:
-// one slot's transfer runs beside the others' copies to the destination.  One
-// set of slots per process (kCopyThreads x kCopySlot), made at the first large
-// copy, used by one call at a time (another call meanwhile takes the plain
-// copy) and handed back by ipg_release_cached_memory.
-constexpr int kCopyThreads = 8;
-constexpr size_t kCopySlot = (size_t)2 << 20;
-struct CopyPool {
-    std::mutex m;
-    int dev = -1;
-    char* slot[kCopyThreads] = {nullptr};
-    hipStream_t st[kCopyThreads] = {nullptr};
-    void release() {
-        for (int t = 0; t < kCopyThreads; t++) {
-            if (slot[t]) (void)hipHostFree(slot[t]);
-            if (st[t]) (void)hipStreamDestroy(st[t]);
-            slot[t] = nullptr;
-            st[t] = nullptr;
-        }
-        dev = -1;
-    }
-    bool ready(int d) {
-        if (dev == d) return true;
-        release();
-        for (int t = 0; t < kCopyThreads; t++)
-            if (hipHostMalloc((void**)&slot[t], kCopySlot, hipHostMallocDefault) != hipSuccess ||
-                hipStreamCreateWithFlags(&st[t], hipStreamNonBlocking) != hipSuccess) {
-                (void)hipGetLastError();
-                release();
-                return false;
-            }
-        dev = d;
-        return true;
-    }
-};
-// never destroyed, as the block cache
-CopyPool& copy_pool() {
-    static CopyPool* p = new CopyPool;
-    return *p;
-}
-// n bytes from device memory, after the work queued on `after`
-hipError_t copy_out(void* dst, const void* src, size_t n, hipStream_t after) {
-    if (n < 2 * kCopySlot) return hipMemcpy(dst, src, n, hipMemcpyDeviceToHost);
-    int dev = 0;
-    hipError_t e = hipGetDevice(&dev);
-    // the slots' streams do not wait for the others by themselves
-    if (e == hipSuccess) e = hipStreamSynchronize(after);
-    if (e != hipSuccess) return e;
-    CopyPool& p = copy_pool();
-    std::unique_lock<std::mutex> lk(p.m, std::try_to_lock);
-    if (!lk.owns_lock() || !p.ready(dev)) return hipMemcpy(dst, src, n, hipMemcpyDeviceToHost);
-    const size_t chunks = (n + kCopySlot - 1) / kCopySlot;
-    const int nt = (int)std::min<size_t>(kCopyThreads, chunks);
-    std::atomic<size_t> next{0};
-    std::atomic<int> err{(int)hipSuccess};
-    auto work = [&](int t) {
-        if (hipSetDevice(dev) != hipSuccess) {
-            err = (int)hipErrorInvalidDevice;
-            return;
-        }
-        for (size_t c = next++; c < chunks && err == (int)hipSuccess; c = next++) {
-            const size_t o = c * kCopySlot, len = std::min(kCopySlot, n - o);
-            hipError_t r = hipMemcpyAsync(p.slot[t], (const char*)src + o, len, hipMemcpyDeviceToHost, p.st[t]);
-            if (r == hipSuccess) r = hipStreamSynchronize(p.st[t]);
-            if (r != hipSuccess) {
-                err = (int)r;
-                return;
-            }
-            std::memcpy((char*)dst + o, p.slot[t], len);
-        }
-    };
-    std::thread th[kCopyThreads];
-    try {
-        for (int t = 1; t < nt; t++) th[t] = std::thread(work, t);
-    } catch (...) {
-        // fewer threads: the others take the chunks
-    }
-    work(0);
-    for (std::thread& x : th)
-        if (x.joinable()) x.join();
-    return (hipError_t)err.load();
 }
 
 // [18][S] planes -> [S][18]
@@ -2018,11 +1933,7 @@ int ipg_release_cached_memory(void) {
     if (have) (void)hipSetDevice(dev);
     c.blocks.clear();
     c.bytes = 0;
-    {
-        CopyPool& p = copy_pool();
-        std::lock_guard<std::mutex> cl(p.m);
-        p.release();
-    }
+    copy_out_release();
     return IPG_OK;
 }
 int ipg_version(void) { return 100; }
