@@ -99,6 +99,11 @@ hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipSt
     st->q.push_back([=] { __builtin_memcpy(d, s, n); });
     return hipSuccess;
 }
+hipError_t hipMemcpyWithStream(void* d, const void* s, size_t n, hipMemcpyKind k, hipStream_t st) {
+    std::lock_guard<std::recursive_mutex> lk(rt);
+    const hipError_t e = hipMemcpyAsync(d, s, n, k, st);
+    return e == hipSuccess ? hipStreamSynchronize(st) : e;
+}
 hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind) {
     std::lock_guard<std::recursive_mutex> lk(rt);
     null_copies++;

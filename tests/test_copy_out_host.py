@@ -55,3 +55,15 @@ def test_pageable_copy_waits_for_its_own_stream_only(lib, k, busy, fail):
 def test_failed_slot_copy_is_reported(lib):
     r = case(lib, 19 * lib.copy_out_slot(), fail=2)
     assert r["status"] == 1 and r["alive"] == 0, r
+
+
+@pytest.mark.parametrize("k", range(6))
+@pytest.mark.parametrize("kind", [PINNED, DEVICE, MANAGED])
+def test_destination_the_device_reaches_takes_one_copy(lib, k, kind):
+    """not the slots, whose memcpy is slower than the DMA into pinned memory and
+    wrong for device memory"""
+    n = sizes(lib)[k]
+    r = case(lib, n, kind=kind)
+    assert r["status"] == 0 and r["right"] == 1 and r["error"] == 0, r
+    assert r["direct"] == n and r["slots"] == 0, r
+    assert r["drained_other"] == 0 and r["null_copies"] == 0, r
