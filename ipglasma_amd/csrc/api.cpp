@@ -897,7 +897,9 @@ struct Engine {
     int fields() {
         const int nev = (int)ev.size();
         ipg_launch_links(d_desc, nev, nblk, st);
-        ipg_launch_newton(d_desc, nev, nlinkblk, d_work, st);
+        bool polish = false;
+        for (const EvDesc& d : desc) polish |= d.active && d.newton_polish > 0;
+        ipg_launch_newton(d_desc, nev, nlinkblk, d_work, polish, st);
         ipg_launch_newton_stats(d_desc, nev, nlinkblk, d_out, st);
         ipg_launch_pi_init(d_desc, nev, nblk, st);
         ipg_launch_zero_fields(d_desc, nev, nblk, st);

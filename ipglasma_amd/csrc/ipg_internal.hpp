@@ -82,8 +82,9 @@ void ipg_launch_unit_v(const EvDesc* d_evs, int nev, int nblk, hipStream_t st);
 
 // tau = 0 fields
 void ipg_launch_links(const EvDesc* d_evs, int nev, int nblk, hipStream_t st);
-// d_cnt: 1 + nev ints of scratch; the events' land_epsv planes hold link lists
-void ipg_launch_newton(const EvDesc* d_evs, int nev, int nlinkblk, int* d_cnt, hipStream_t st);
+// d_cnt: 1 + nev ints of scratch; the events' land_epsv planes hold link lists;
+// polish: some event has newton_polish > 0
+void ipg_launch_newton(const EvDesc* d_evs, int nev, int nlinkblk, int* d_cnt, bool polish, hipStream_t st);
 void ipg_launch_newton_stats(const EvDesc* d_evs, int nev, int nlinkblk, double* d_out, hipStream_t st);
 void ipg_launch_pi_init(const EvDesc* d_evs, int nev, int nblk, hipStream_t st);
 void ipg_launch_zero_fields(const EvDesc* d_evs, int nev, int nblk, hipStream_t st);

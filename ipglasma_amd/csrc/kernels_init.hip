@@ -9,7 +9,8 @@
 //                 inverse FFT, V <- exp(-i A.t) V  (Init.cpp:1678-1850)
 //   k_links       U^(1,2)_{x,y} = V(x) V(x+i)^+ with the NaN guard
 //                 (Init.cpp:2459-2491)
-//   k_newton_quad, k_newton  per-link root finder (Init.cpp:3344-3481)
+//   k_newton_quad, k_newton, k_newton_polish  per-link root finder
+//                 (Init.cpp:3344-3481)
 //   k_pi_init     pi = -(2i/g) A^eta (Init.cpp:2521-2584, 2664-2680)
 #include <algorithm>
 
@@ -1056,9 +1057,9 @@ __device__ __forceinline__ void solve_rows(double (&J)[64], double (&F)[8]) {
 // every lane solves it in registers.  The first iteration starts from exponent
 // 0 at every link, so its column exponentials are the same everywhere and come
 // from a table.  Almost every link converges in two to six iterations (mean
-// 2.1 to 4.0 over the lattices in use); one that has not after kQuadIter, that
-// wants a restart, or that polishes goes to its event's list for k_newton,
-// which starts it afresh.
+// 2.1 to 4.0 over the lattices in use); one that has not after kQuadIter, or
+// that wants a restart, goes to its event's list for k_newton, which starts it
+// afresh.
 // FP64 issue bounds it, most of it in the exponentials.  N = 512 (2.1
 // iterations a link) / N = 128 (3.2): eight lanes a link, all of them repeating
 // the residual, the update and its exponential, with the elimination by
@@ -1082,7 +1083,6 @@ __global__ __launch_bounds__(64, 2) void k_newton_quad(const EvDesc* __restrict_
     if (l - k >= 2 * S) return;
     const int dir = l >= S;
     const long long s = dir ? l - S : l;
-    const bool direct = ev.newton_polish == 0;
     auto ld = [&](const double (*m)[kQuadLinks]) {
         // read where used: kept in registers across the loops they spill
         asm volatile("" ::: "memory");
@@ -1101,28 +1101,26 @@ __global__ __launch_bounds__(64, 2) void k_newton_quad(const EvDesc* __restrict_
     double alpha[8];
 #pragma unroll
     for (int a = 0; a < 8; a++) alpha[a] = 0.;
-    if (direct) {
-        if (lane < 8) {
-            double p[8];
-            (void)column_exponent(alpha, lane, p);
-            const M3 E = exp_iQt(p);
+    if (lane < 8) {
+        double p[8];
+        (void)column_exponent(alpha, lane, p);
+        const M3 E = exp_iQt(p);
 #pragma unroll
-            for (int q = 0; q < 9; q++) {
-                tab[lane][2 * q] = E.e[q].r;
-                tab[lane][2 * q + 1] = E.e[q].i;
-            }
-        }
-        const M3 U1 = ldm(dir ? ev.L1y : ev.L1x, S, s);
-        const M3 U2 = ldm(dir ? ev.L2y : ev.L2x, S, s);
-        if (sub == 0) {
-            const M3 U0 = U1 * U2;
-            st(mU0, U0);
-            st(mW, U1 + U2);
-            // exp(0) is the identity (its closed form gives no number, the guard 1)
-            st(mUs, U0);
+        for (int q = 0; q < 9; q++) {
+            tab[lane][2 * q] = E.e[q].r;
+            tab[lane][2 * q + 1] = E.e[q].i;
         }
     }
-    bool done = !direct, failed = !direct;
+    const M3 U1 = ldm(dir ? ev.L1y : ev.L1x, S, s);
+    const M3 U2 = ldm(dir ? ev.L2y : ev.L2x, S, s);
+    if (sub == 0) {
+        const M3 U0 = U1 * U2;
+        st(mU0, U0);
+        st(mW, U1 + U2);
+        // exp(0) is the identity (its closed form gives no number, the guard 1)
+        st(mUs, U0);
+    }
+    bool done = false, failed = false;
     int analytic = 0;
     __syncthreads();
     for (int iter = 1; iter <= kQuadIter && __any(!done); iter++) {
@@ -1269,7 +1267,7 @@ __global__ __launch_bounds__(NWB, 1) void k_newton(const EvDesc* __restrict__ ev
 #pragma unroll
     for (int a = 0; a < 8; a++) alpha[a] = 0.;
     double Fzero = 0., Fmin = 0.;
-    int iter = 0, nRestart = 0, total = 0, analytic = 0, best_one = 1, npol = 0;
+    int iter = 0, nRestart = 0, total = 0, analytic = 0, best_one = 1;
     uint32_t ndraw = 0;
     if (c == 0) {
         lds_st(mU0, m_one());
@@ -1323,7 +1321,7 @@ __global__ __launch_bounds__(NWB, 1) void k_newton(const EvDesc* __restrict__ ev
                         best_one = 1;
                         Fzero = 10.;
                         Fmin = 1e6;
-                        iter = nRestart = total = analytic = npol = 0;
+                        iter = nRestart = total = analytic = 0;
                         ndraw = 0;
                         state = 1;
                     }
@@ -1345,27 +1343,16 @@ __global__ __launch_bounds__(NWB, 1) void k_newton(const EvDesc* __restrict__ ev
             Fzero = residual(lds_m3(mW), lds_m3(mUs), tr8, F);
         }
         double col[8];
-        bool good = true;
-        if (npol == 0) {
-            double p[8];
-            const double d = column_exponent(alpha, c, p);
-            good = jacobian_column(lds_m3(mW), dag(exp_iQt(p) * lds_m3(mU0)) - dag(lds_m3(mUs)), d, col);
+        double p[8];
+        const double d = column_exponent(alpha, c, p);
+        const bool good = jacobian_column(lds_m3(mW), dag(exp_iQt(p) * lds_m3(mU0)) - dag(lds_m3(mUs)), d, col);
 #pragma unroll
-            for (int k = 0; k < 8; k++) {
-                const double dk = fmax(0.001, fmin(10., 0.01 * fabs(alpha[k])));
-                alpha[k] = (alpha[k] + dk) - dk;
-            }
-        } else {
-            // newton_polish: the exact Jacobian about the iterate,
-            // U <- exp(i beta^a t^a) U, J_ab = -2 Re tr(t^a W U^+ t^b)
-            const M3 X = dag(gen_mul(c, mul_bd(lds_m3(mUs), lds_m3(mW))));
-            cd t[8];
-            tr_gen(X, t);
-#pragma unroll
-            for (int a = 0; a < 8; a++) col[a] = -2. * t[a].r;
+        for (int k = 0; k < 8; k++) {
+            const double dk = fmax(0.001, fmin(10., 0.01 * fabs(alpha[k])));
+            alpha[k] = (alpha[k] + dk) - dk;
         }
         const unsigned long long bad = __ballot(!good);
-        if (npol == 0 && ((bad >> (grp * NG)) & 0xFFull)) {
+        if ((bad >> (grp * NG)) & 0xFFull) {
             analytic = 1;
             analytic_column(lds_m3(mW), lds_m3(mUs), c, col);
         }
@@ -1383,41 +1370,28 @@ __global__ __launch_bounds__(NWB, 1) void k_newton(const EvDesc* __restrict__ ev
 #pragma unroll
         for (int a = 0; a < 8; a++)
             if (fabs(y[a]) > 1e5) okstep = false;
-        if (npol == 0) {
-            if (okstep) {
+        if (okstep) {
 #pragma unroll
-                for (int a = 0; a < 8; a++) alpha[a] = alpha[a] + y[a];
-            } else {
-                restart_alpha(evs[e].newton_seed, link, ndraw++, alpha);
-            }
-            if (Fzero < Fmin) {
-                // best = the new iterate, kept as its exponent (Us is exp(i alpha t) U0)
-                Fmin = Fzero;
-                if (c == 0)
-#pragma unroll
-                    for (int a = 0; a < 8; a++) best_alpha[a] = alpha[a];
-                best_one = 0;
-            }
-            if (iter == maxIt) {
-                restart_alpha(evs[e].newton_seed, link, ndraw++, alpha);
-                nRestart++;
-                iter = 0;
-            }
+            for (int a = 0; a < 8; a++) alpha[a] = alpha[a] + y[a];
+        } else {
+            restart_alpha(evs[e].newton_seed, link, ndraw++, alpha);
         }
-        M3 Us;
-        {
-            double q[8];
+        if (Fzero < Fmin) {
+            // best = the new iterate, kept as its exponent (Us is exp(i alpha t) U0)
+            Fmin = Fzero;
+            if (c == 0)
 #pragma unroll
-            for (int a = 0; a < 8; a++) q[a] = npol > 0 ? y[a] : alpha[a];
-            Us = exp_iQt(q) * lds_m3(npol > 0 ? mUs : mU0);
+                for (int a = 0; a < 8; a++) best_alpha[a] = alpha[a];
+            best_one = 0;
         }
+        if (iter == maxIt) {
+            restart_alpha(evs[e].newton_seed, link, ndraw++, alpha);
+            nRestart++;
+            iter = 0;
+        }
+        M3 Us = exp_iQt(alpha) * lds_m3(mU0);
         if (c == 0) lds_st(mUs, Us);
-        bool stop = state == 1 && !(Fzero > 1e-6 && iter < maxIt && nRestart < maxRe);
-        // optional exact Newton steps of a converged link (newton_polish)
-        if (stop && nRestart != maxRe && (Fzero <= 1e-6 || npol > 0) && npol < evs[e].newton_polish) {
-            npol++;
-            stop = false;
-        }
+        const bool stop = state == 1 && !(Fzero > 1e-6 && iter < maxIt && nRestart < maxRe);
         if (stop) {
             const EvDesc& ev = evs[e];
             const int conv = nRestart != maxRe;
@@ -1433,6 +1407,54 @@ __global__ __launch_bounds__(NWB, 1) void k_newton(const EvDesc* __restrict__ ev
         }
         __syncthreads();  // Us, best exponent visible before the next round
     }
+}
+
+// newton_polish: exact Newton steps of the converged links, U <- exp(i y^a t^a) U
+// with J_ab = -2 Re tr(t^a W U^+ t^b) about U.  A lane a link, everything in
+// registers: no work is repeated and every link takes the same steps (in
+// k_newton, where the polishing links were, eight lanes repeat the elimination
+// and the exponential of a link and no more than 1024 wavefronts run: the tau = 0
+// fields with four steps took 7.8 ms at N = 512 and 2.5 at N = 256; with this
+// kernel 1.31 and 0.50, without steps 1.15 and 0.46).
+__global__ __launch_bounds__(NWB, 1) void k_newton_polish(const EvDesc* __restrict__ evs, int nev) {
+    const int e = find_event_links(evs, nev, blockIdx.x);
+    const EvDesc& ev = evs[e];
+    if (!ev.active || ev.newton_polish == 0) return;
+    const long long S = ev.S;
+    const long long l = ((long long)blockIdx.x - ev.lblock0) * NWB + threadIdx.x;
+    if (l >= 2 * S) return;
+    const int dir = l >= S;
+    const long long s = dir ? l - S : l;
+    const int stat = ev.newton_stat[l];
+    if (stat & (1 << 28)) return;  // no root found
+    const M3 W = ldm(dir ? ev.L1y : ev.L1x, S, s) + ldm(dir ? ev.L2y : ev.L2x, S, s);
+    M3 Us = ldm(ev.U[0][dir], S, s);
+    double trci[8];
+    {
+        cd trc[8];
+        tr_gen(W - dag(W), trc);
+#pragma unroll
+        for (int a = 0; a < 8; a++) trci[a] = trc[a].i;
+    }
+    // a step that finds the residual above the stopping level is not counted
+    int total = 0;
+    for (int n = 0; n < ev.newton_polish && total < 2000; total++) {
+        double F[8];
+        if (!(residual(W, Us, trci, F) > 1e-6)) n++;
+        const M3 UW = mul_bd(Us, W);
+        double J[64];
+#pragma unroll
+        for (int c = 0; c < 8; c++) {
+            cd t[8];
+            tr_gen(dag(gen_mul(c, UW)), t);
+#pragma unroll
+            for (int a = 0; a < 8; a++) J[8 * a + c] = -2. * t[a].r;
+        }
+        solve_rows(J, F);
+        Us = exp_iQt(F) * Us;
+    }
+    stm(ev.U[0][dir], S, s, Us);
+    ev.newton_stat[l] = stat + total;
 }
 
 // A^eta from the four links touching the site, pi = -(2i/g) A^eta
@@ -1644,10 +1666,11 @@ __global__ void k_zero_counters(int* c, int n) {
 
 // d_cnt: 1 + nev ints.  The second pass is persistent: enough one-wave blocks
 // for a wave on every SIMD (256 CUs x 4); each loops until the lists run out.
-void ipg_launch_newton(const EvDesc* d, int nev, int nlinkblk, int* d_cnt, hipStream_t st) {
+void ipg_launch_newton(const EvDesc* d, int nev, int nlinkblk, int* d_cnt, bool polish, hipStream_t st) {
     hipLaunchKernelGGL(k_zero_counters, dim3((unsigned)(nev + 1 + 255) / 256), dim3(256), 0, st, d_cnt, nev + 1);
     hipLaunchKernelGGL(k_newton_quad, dim3(NWB / kQuadLinks * nlinkblk), dim3(NWB), 0, st, d, nev, d_cnt);
     hipLaunchKernelGGL(k_newton, dim3(std::min(1024, nlinkblk)), dim3(NWB), 0, st, d, nev, d_cnt);
+    if (polish) hipLaunchKernelGGL(k_newton_polish, dim3(nlinkblk), dim3(NWB), 0, st, d, nev);
 }
 
 // per event: sum, max of the link iteration counts, restarts, unconverged
