@@ -1451,7 +1451,7 @@ __global__ __launch_bounds__(NWB, 1) void k_newton_polish(const EvDesc* __restri
             for (int a = 0; a < 8; a++) J[8 * a + c] = -2. * t[a].r;
         }
         solve_rows(J, F);
-        Us = exp_iQt(F) * Us;
+        Us = exp_step(F) * Us;
     }
     stm(ev.U[0][dir], S, s, Us);
     ev.newton_stat[l] = stat + total;

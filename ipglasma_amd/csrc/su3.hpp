@@ -681,6 +681,31 @@ IPG_HD M3 exp_iQt(const double Q[8]) {
     return U;
 }
 
+// exp(i Q^a t^a) for the root finder's polishing steps.  Below c1 = tr(Q.t)^2/2
+// = 1e-8 the closed form's f_j are differences of numbers c1 times smaller than
+// their terms: its error reaches the size of Q at Q ~ 1e-8, and from ~1e-8 down
+// its f_2 is 0 or its guard takes the identity, so that a step did nothing.
+// There the series to third order leaves 1e-17.
+IPG_HD M3 exp_step(const double Q[8]) {
+    double c1 = 0.;
+#pragma unroll
+    for (int a = 0; a < 8; a++) c1 += Q[a] * Q[a];
+    if (!(0.25 * c1 < 1e-8)) return exp_iQt(Q);
+    const double s3 = 1.0 / (2.0 * sqrt(3.0));
+    M3 X;
+    X.e[0] = cd{0., 0.5 * Q[2] + s3 * Q[7]};
+    X.e[1] = cd{0.5 * Q[1], 0.5 * Q[0]};
+    X.e[2] = cd{0.5 * Q[4], 0.5 * Q[3]};
+    X.e[3] = cd{-0.5 * Q[1], 0.5 * Q[0]};
+    X.e[4] = cd{0., s3 * Q[7] - 0.5 * Q[2]};
+    X.e[5] = cd{0.5 * Q[6], 0.5 * Q[5]};
+    X.e[6] = cd{-0.5 * Q[4], 0.5 * Q[3]};
+    X.e[7] = cd{-0.5 * Q[6], 0.5 * Q[5]};
+    X.e[8] = cd{0., -2. * s3 * Q[7]};
+    const M3 X2 = X * X;
+    return m_one() + X + 0.5 * X2 + (1. / 6.) * (X2 * X);
+}
+
 // t^a (Group.cpp:68-149) applied on the left: (t^a M)
 IPG_HD M3 gen_mul(int a, const M3& M) {
     M3 c = m_zero();

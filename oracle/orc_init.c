@@ -143,6 +143,29 @@ static void solve8(double *J /* row-major 8x8, destroyed */, const double *F, do
  * converges quadratically (the reference's forward-difference Jacobian in
  * alpha, with steps of at least 1e-3, does not converge past ~1e-9). */
 static int newton_polish = 0;
+
+/* exp(i beta^a t^a) of a polishing step.  The closed form's coefficients are
+ * differences of nearly equal numbers for a small exponent (its error is the
+ * exponent's own size at ~1e-8, and below that it returns the identity), so
+ * there the series is summed: X^4/24 is below 1e-17 where c1 < 1e-8. */
+static M3 polish_exp(const double b[8], const M3 t[8]) {
+    double c1 = 0.;
+    for (int a = 0; a < 8; a++) c1 += 0.25 * b[a] * b[a];
+    if (!(c1 < 1e-8)) return orc_exp_iQt(b);
+    M3 X;
+    for (int k = 0; k < 9; k++) {
+        X.e[k] = 0.;
+        for (int a = 0; a < 8; a++) X.e[k] += CMPLX(0., b[a]) * t[a].e[k];
+    }
+    M3 U = m_one(), P = m_one();
+    for (int n = 1; n <= 3; n++) {
+        P = m_mul(P, X);
+        for (int k = 0; k < 9; k++) P.e[k] /= n;
+        U = m_add(U, P);
+    }
+    return U;
+}
+
 void orc_set_newton_polish(int n) { newton_polish = n < 0 ? 0 : n; }
 
 int orc_newton_link(const double *pU1, const double *pU2, uint64_t seed, uint32_t link,
@@ -188,7 +211,7 @@ int orc_newton_link(const double *pU1, const double *pU2, uint64_t seed, uint32_
                 for (int a = 0; a < 8; a++) Jab[8 * a + b] = -2. * creal(m_trprod(t[a], X));
             }
             solve8(Jab, Fa, dal);
-            Usol = m_mul(orc_exp_iQt(dal), Usol);
+            Usol = m_mul(polish_exp(dal, t), Usol);
             Ud = m_dag(Usol);
             continue;
         }

@@ -6,6 +6,8 @@ import numpy as np
 import pytest
 
 import _cases as K
+import _oracle as O
+from test_gpu_parity import _GEN
 
 pytestmark = pytest.mark.gpu
 
@@ -40,6 +42,30 @@ def test_polish_goes_on_from_the_plain_iterate(system, N):
             # Sum|F| <= 1e-6 and a Jacobian near the identity where links are near 1
             assert np.abs(ev.field(k) - u)[f].max() < 1e-5
         ev.close()
+
+
+@pytest.mark.parametrize("system,N", [("pPb", 32), ("AuAu", 32), ("OO", 64)])
+def test_polish_takes_links_to_round_off(system, N):
+    """Sum|F_a| below 1e-13, the oracle's own bound: F is eight traces of products
+    of matrices of norm 2 at most, ~5e-15 of round-off each way.  Four steps from
+    1e-6 do it wherever the Jacobian's inverse is below ~100 (each step squares
+    the distance, 1e-4 at most, up to a factor of that size)"""
+    ev = _event(system, N, 5, newton_polish=4)
+    S, idx = N * N, np.arange(N * N)
+    V = [O.from_c(ev.field(k)) for k in ("VA", "VB")]
+    nb = {"Ux": np.minimum(idx // N + 1, N - 1) * N + idx % N, "Uy": idx // N * N + np.minimum(idx % N + 1, N - 1)}
+    for k, n in nb.items():
+        U = O.from_c(ev.field(k))
+        W = sum(v @ v[n].conj().transpose(0, 2, 1) for v in V)
+        WU = W @ U.conj().transpose(0, 2, 1)
+        M = W - W.conj().transpose(0, 2, 1) + WU - WU.conj().transpose(0, 2, 1)
+        F = np.stack([-np.imag(np.trace(t @ M, axis1=1, axis2=2)) for t in _GEN], 1)
+        J = np.stack([np.stack([-2 * np.real(np.trace(t @ WU @ u, axis1=1, axis2=2)) for u in _GEN], 1)
+                      for t in _GEN], 1)
+        fine = np.linalg.svd(J, compute_uv=False)[:, -1] > 0.01
+        assert fine.mean() > 0.5
+        assert np.abs(F).sum(1)[fine].max() < 1e-13, (k, np.sort(np.abs(F).sum(1)[fine])[-5:])
+    ev.close()
 
 
 def test_events_of_a_batch_polish_each_by_its_own_count():
