@@ -17,6 +17,7 @@
 #include "ipg_device.hpp"
 #include "ipg_internal.hpp"
 #include "fft_lds.hpp"
+#include "solve_rows.hpp"
 #include "adjoint.hpp"
 
 namespace {
@@ -1005,53 +1006,6 @@ __device__ __forceinline__ void analytic_column(const M3& W, const M3& Us, int c
 #pragma unroll
     for (int a = 0; a < 8; a++) col[a] = -2. * retrprod(gen_mul(a, W), Mb);
 }
-// J y = F by Gaussian elimination with partial pivoting (first maximal pivot),
-// J row-major, in registers; y replaces F.  Rows are exchanged by selects, and
-// only when some lane of the wavefront has an exchange to make.
-__device__ __forceinline__ void solve_rows(double (&J)[64], double (&F)[8]) {
-#pragma unroll
-    for (int j = 0; j < 7; j++) {
-        double best = fabs(J[9 * j]);
-        int p = j;
-#pragma unroll
-        for (int r = j + 1; r < 8; r++)
-            if (fabs(J[8 * r + j]) > best) {
-                best = fabs(J[8 * r + j]);
-                p = r;
-            }
-        if (__any(p != j)) {
-#pragma unroll
-            for (int r = j + 1; r < 8; r++) {
-                const bool sw = r == p;
-#pragma unroll
-                for (int c = j; c < 8; c++) {
-                    const double x = J[8 * j + c], y = J[8 * r + c];
-                    J[8 * j + c] = sw ? y : x;
-                    J[8 * r + c] = sw ? x : y;
-                }
-                const double x = F[j], y = F[r];
-                F[j] = sw ? y : x;
-                F[r] = sw ? x : y;
-            }
-        }
-        const double inv = J[9 * j] != 0. ? 1. / J[9 * j] : 0.;
-#pragma unroll
-        for (int r = j + 1; r < 8; r++) {
-            const double f = J[8 * r + j] * inv;
-#pragma unroll
-            for (int c = j + 1; c < 8; c++) J[8 * r + c] -= f * J[8 * j + c];
-            F[r] -= f * F[j];
-        }
-    }
-#pragma unroll
-    for (int r = 7; r >= 0; r--) {
-        double t = F[r];
-#pragma unroll
-        for (int c = r + 1; c < 8; c++) t -= J[8 * r + c] * F[c];
-        F[r] = t / J[9 * r];
-    }
-}
-
 // First pass of the root finder: four lanes per link, 16 links a wavefront.
 // Each lane evaluates two Jacobian columns; the system goes through LDS and
 // every lane solves it in registers.  The first iteration starts from exponent
