@@ -29,8 +29,10 @@ Printed JSON fields beyond metric, value, unit, steps, config and the timing key
                       value) and Au+Au N=256, with the CPU model
 """
 import argparse
+import hashlib
 import json
 import os
+import re
 import sys
 import time
 
@@ -260,17 +262,32 @@ def run_batched(I, p, seeds, use_graph=True):
     return time.perf_counter() - t0, out
 
 
+TRAFFIC_PROFILE = os.path.join(ROOT, "profiles", "k_step_pbpb_n512_hbm_traffic.md")
+
+
+def k_step_fingerprint():
+    """Hash of k_step's source without comments and blanks: which kernel a
+    committed counter figure belongs to."""
+    src = open(os.path.join(ROOT, "ipglasma_amd", "csrc", "kernels_evolve.hip")).read()
+    a = src.rindex("__global__", 0, src.index("void k_step("))
+    body = re.sub(r"//[^\n]*", "", src[a:src.index("\n}\n", a)])
+    return hashlib.sha256("".join(body.split()).encode()).hexdigest()[:16]
+
+
 def measured_traffic(N):
     """HBM bytes per k_step launch from the committed FETCH_SIZE/WRITE_SIZE
-    counter passes (profiles/k_step_pbpb_n512_hbm_traffic.md); None for
-    other sizes."""
-    f = os.path.join(ROOT, "profiles", "k_step_pbpb_n512_hbm_traffic.md")
-    if N != 512 or not os.path.exists(f):
+    counter passes; None for other sizes, and where they counted another
+    k_step than the present one."""
+    if N != 512 or not os.path.exists(TRAFFIC_PROFILE):
         return None
-    for line in open(f):
-        if line.startswith("traffic_bytes_per_launch:"):
-            return int(line.split(":")[1])
-    return None
+    v = {}
+    for line in open(TRAFFIC_PROFILE):
+        k, _, x = line.partition(":")
+        if k in ("traffic_bytes_per_launch", "traffic_kernel"):
+            v[k] = x.strip()
+    if v.get("traffic_kernel") != k_step_fingerprint():
+        return None
+    return int(v["traffic_bytes_per_launch"])
 
 
 def roofline(I, p):
