@@ -99,7 +99,8 @@ def _init_to_fields(p, seed):
     return ev
 
 
-@pytest.mark.parametrize("system,N,seed", [("AuAu", 32, 5), ("pPb", 32, 2), ("AuAu", 48, 5), ("PbPb", 96, 7)])
+@pytest.mark.parametrize("system,N,seed", [("AuAu", 32, 5), ("pPb", 32, 2), ("AuAu", 48, 5), ("PbPb", 96, 7),
+                                           ("pPb", 128, 2), ("OO", 192, 4)])
 def test_wilson_lines(system, N, seed):
     p = K.params(system, N=N, Ny=3)
     ev = _init_to_fields(p, seed)
@@ -350,14 +351,17 @@ def test_step_builds_agree():
         np.testing.assert_allclose(o[k], plain[k], rtol=1e-11, atol=1e-13, err_msg=k)
 
 
-@pytest.mark.parametrize("system,N,Ny", [("AuAu", 256, 6), ("PbPb", 512, 5)])
+@pytest.mark.parametrize("system,N,Ny", [("AuAu", 256, 6), ("PbPb", 512, 5), ("AuAu", 16, 5), ("AuAu", 48, 6),
+                                         ("AuAu", 96, 5), ("pPb", 128, 7), ("OO", 192, 5)])
 def test_setv_launch_shapes_agree(system, N, Ny):
     """One chunk of Ny slices: while the tuner measures the six inverse-row
     launch shapes (256- and 512-thread blocks, each also with the next slice
-    prefetched into registers and with the twiddles in LDS), the four
-    forward-row and the three column shapes, three runs each, repeated
-    initialisations of one event give the same Wilson lines bit for bit (the
-    same arithmetic per site)"""
+    prefetched into registers and with the twiddles in LDS), the three column
+    shapes and, from N = 256 on, the four forward-row shapes, three runs each,
+    repeated initialisations of one event give the same Wilson lines bit for
+    bit (the same arithmetic per site).  Below N = 256 the forward row pass
+    takes several lattice rows a block: 16 at N = 16, 4 at 48, 2 at 96 and 128,
+    1 at 192, the 3 2^a lengths among them."""
     import ipglasma_amd as I
     p = K.params(system, N=N, Ny=Ny)
     key = f"setv_rows_inv_block/N={N}/events=1/kc={Ny}"
@@ -386,8 +390,13 @@ def test_setv_launch_shapes_agree(system, N, Ny):
             for a, b in zip(V, ref):
                 np.testing.assert_array_equal(a, b, err_msg=f"run {run}")
     rep = I.autotune_report()
-    assert key in rep and len(rep[key]["times_ms"]) == 6, rep.get(key)
-    assert all(t > 0 for t in rep[key]["times_ms"]), rep[key]
+    shapes = {"inv": ("setv_rows_inv_block", 6), "cols": ("setv_cols_block", 3)}
+    if N >= 256:
+        shapes["fwd"] = ("setv_rows_fwd_block", 4)
+    for name, n in shapes.values():
+        key = f"{name}/N={N}/events=1/kc={Ny}"
+        assert key in rep and len(rep[key]["times_ms"]) == n, rep.get(key)
+        assert all(t > 0 for t in rep[key]["times_ms"]), rep[key]
 
 
 def test_full_size_pbpb_event_invariants():
