@@ -291,7 +291,7 @@ def measured_traffic(N):
 
 
 def roofline(I, p):
-    # one untimed event first: the autotuner settles the step kernel's build
+    # one untimed event first: the autotuner settles the step kernel's block order
     w = I.Event(p, seed=12344)
     while not w.init():
         pass

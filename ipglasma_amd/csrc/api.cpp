@@ -353,8 +353,8 @@ struct Engine {
     hipGraphExec_t gexec[3] = {nullptr, nullptr, nullptr};
     int graph_itm[3] = {-1, -1, -1};
     std::vector<int> graph_act[3];  // active flags the graph was captured with
-    int graph_var[3] = {-1, -1, -1};  // k_step build the graph was captured with
-    int step_var = 0;                 // k_step build for launches not being timed
+    int graph_var[3] = {-1, -1, -1};  // k_step block order the graph was captured with
+    int step_var = 0;                 // k_step block order for launches not being timed
     // reverse-mode workspace (checkpoints, cotangents, the rho gradient),
     // kept between calls; grown on demand
     double* adj_ws = nullptr;
@@ -842,8 +842,7 @@ struct Engine {
             int minNy = 1 << 30;
             for (int e : es) minNy = std::min(minNy, desc[e].Ny);
             auto chunk = [&](const EvDesc* dd, int n, int k0, int kcc, int ny) {
-                // keyed by the launch's own event count and chunk length; the
-                // forward row pass has candidates from N = 256 on
+                // keyed by the launch's own event count and chunk length
                 const std::string tail = "/N=" + std::to_string(kv.first) + "/events=" + std::to_string(n) +
                                          "/kc=" + std::to_string(kcc);
                 SetvVariant v;
@@ -853,17 +852,16 @@ struct Engine {
                 const bool full = k0 + kcc <= ny;
                 v.inv = g_tuner.pick("setv_rows_inv_block" + tail, 6, &meas);
                 timed_begin("setv_rows_inv_block" + tail, v.inv, meas && full, &t.inv[0], &t.inv[1]);
+                // 0: 256-thread blocks, 1: 512-thread blocks, 2: one wavefront per
+                // transformed row or column, synchronised alone (forward rows
+                // 3: 2 with the twiddles in LDS); below N = 256 the forward
+                // rows have one form, several lattice rows a block
                 if (kv.first >= 256) {
-                    // 0: 256-thread blocks, 1: 512-thread blocks, 2: one
-                    // wavefront per transformed row, synchronised alone
-                    // (forward rows 3: 2 with the twiddles in LDS)
                     v.fwd = g_tuner.pick("setv_rows_fwd_block" + tail, 4, &meas);
                     timed_begin("setv_rows_fwd_block" + tail, v.fwd, meas && full, &t.fwd[0], &t.fwd[1]);
                 }
-                {
-                    v.cols = g_tuner.pick("setv_cols_block" + tail, 3, &meas);
-                    timed_begin("setv_cols_block" + tail, v.cols, meas && full, &t.cols[0], &t.cols[1]);
-                }
+                v.cols = g_tuner.pick("setv_cols_block" + tail, 3, &meas);
+                timed_begin("setv_cols_block" + tail, v.cols, meas && full, &t.cols[0], &t.cols[1]);
                 ipg_launch_setv_chunk(dd, n, dp, k0, kcc, v, t, st);
             };
             // schedule (a tuner choice when several events share the size):
@@ -937,7 +935,7 @@ struct Engine {
         return false;
     }
 
-    // tuner key of the k_step build (waves per SIMD) for the active events
+    // tuner key of k_step's block order for the active events
     std::string step_key() const {
         int nact = 0, maxN = 0;
         for (const EvDesc& d : desc)
@@ -945,7 +943,7 @@ struct Engine {
                 nact++;
                 maxN = std::max(maxN, d.N);
             }
-        return "step_waves_per_simd/N=" + std::to_string(maxN) + "/events=" + std::to_string(nact);
+        return "step_block_order/N=" + std::to_string(maxN) + "/events=" + std::to_string(nact);
     }
     int step_decided() const { return std::max(0, g_tuner.chosen(step_key())); }
 

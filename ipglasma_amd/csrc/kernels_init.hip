@@ -373,9 +373,9 @@ __global__ __launch_bounds__(IPG_BLOCK) void k_stats(const EvDesc* __restrict__ 
     const int lb = xcd_remap(blockIdx.x - ev.block0, ev.nblocks);
     const long long s = (long long)lb * IPG_BLOCK + threadIdx.x;
     // the wounded nucleons within rcut of the block's sites (a superset, by the
-    // rows and, inside one row, the columns it covers); the loop over all of them per site was 130 us of the
-    // kernel's 146 at N = 512 with 416 nucleons.  A list that would not fit
-    // falls back to that loop.
+    // rows and, inside one row, the columns it covers); the loop over all of
+    // them per site was 130 us of the kernel's 146 at N = 512 with 416
+    // nucleons.  A list that would not fit falls back to that loop.
     __shared__ int near_idx[2][kNearCap];
     __shared__ int near_n[2];
     if (threadIdx.x < 2) near_n[threadIdx.x] = 0;
@@ -1017,8 +1017,9 @@ __device__ __forceinline__ void analytic_column(const M3& W, const M3& Us, int c
 // FP64 issue bounds it, most of it in the exponentials.  N = 512 (2.1
 // iterations a link) / N = 128 (3.2): eight lanes a link, all of them repeating
 // the residual, the update and its exponential, with the elimination by
-// shuffles 1740 / 380 us; this 1020 + 244 / 98 + 9 us (both passes).  Two lanes a link with the columns in
-// registers is less work, but spills at two waves per SIMD (1324 / 190 us).
+// shuffles 1740 / 380 us; this 1020 + 244 / 98 + 9 us (both passes).  Two
+// lanes a link with the columns in registers is less work, but spills at two
+// waves per SIMD (1324 / 190 us).
 constexpr int kQuadIter = 8;
 constexpr int kQuadLinks = 16;
 __global__ __launch_bounds__(64, 2) void k_newton_quad(const EvDesc* __restrict__ evs, int nev, int* __restrict__ cnt) {
@@ -1485,9 +1486,10 @@ void ipg_launch_stats(const EvDesc* d, int nev, int nblk, double* out, hipStream
 // to 128 registers, four waves per SIMD).  Below N = 256 the forward row pass
 // takes several lattice rows a block (the inverse one, serial in the slices,
 // keeps one: two rows a block left half of the CUs without a block, 28 -> 37
-// us a chunk at N = 128).  Each pass is bracketed by its
-// pair of events when they are given.
-// the column pass in the launch shape of variant cv 
+// us a chunk at N = 128).  Each pass is bracketed by its pair of events when
+// they are given.
+
+// the column pass in the launch shape of variant cv
 template <int N>
 static void launch_cols(const EvDesc* d, const FftPlanDev& pl, int k0, int kc, int ncol, int cv, hipStream_t st) {
     constexpr int C = ipgfft::cols_per_block(N);

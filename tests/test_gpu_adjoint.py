@@ -298,10 +298,11 @@ def test_batched_adjoint_matches_single_event_contexts():
 
 
 def test_reverse_step_kernels_agree():
-    """the reverse leapfrog step as three kernels (tuning off) and, while the
-    tuner measures them, alternating with the fused forms, then
-    with the tuner's choice: the same arithmetic per site, so the gradients
-    agree to the round-off of the loss's atomic sums"""
+    """the gather of a reverse leapfrog step with the local updates of the step
+    before it as one kernel (tuning off) and, while the tuner measures them,
+    alternating with the two kernels, then with the tuner's choice: the same
+    arithmetic per site, so the gradients agree to the round-off of the loss's
+    atomic sums"""
     import os
 
     import ipglasma_amd as I

@@ -4,7 +4,7 @@ field set on the device comes back bit for bit; and from several threads at
 once, of which one gets the pinned slots and the others the plain copy; and
 into pinned and into device memory, which take the plain copy at any size."""
 import ctypes as C
-import threading
+from concurrent.futures import ThreadPoolExecutor
 
 import numpy as np
 import pytest
@@ -31,23 +31,20 @@ def test_field_round_trip(N):
 
 def test_field_round_trip_from_threads():
     import ipglasma_amd as I
-    bad = []
 
     def go(k):
         ev = _event(256)
         a = np.random.default_rng(k).normal(size=(256 * 256, 18))
+        right = 0
         for _ in range(5):
             ev.set_field("Ux", a)
-            if not np.array_equal(ev.field("Ux"), a):
-                bad.append(k)
+            right += np.array_equal(ev.field("Ux"), a)
         ev.close()
+        return right
 
-    th = [threading.Thread(target=go, args=(k,)) for k in range(4)]
-    for t in th:
-        t.start()
-    for t in th:
-        t.join()
-    assert not bad
+    with ThreadPoolExecutor(4) as pool:
+        # result() raises what a thread raised
+        assert [f.result() for f in [pool.submit(go, k) for k in range(4)]] == [5] * 4
     I.release_cached_memory()  # hands the slots back; the next copy makes them again
     test_field_round_trip(192)
 

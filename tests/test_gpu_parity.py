@@ -322,15 +322,16 @@ def test_batch_setv_schedules_match_plain():
     assert "setv_schedule/N=32/events=3" in I.autotune_report()
 
 
-def test_step_builds_agree():
-    """N a multiple of 64: while the tuner measures the four k_step builds
-    (one or two waves per SIMD; 4 x 64 site tiles along y or down column
-    strips) a one-event batch runs them in turn, three steps each; the plain
-    event before it runs the first build throughout.  Same arithmetic per
-    site, so the observables agree to round-off of the reductions."""
+def test_step_block_orders_agree():
+    """N a multiple of 64: while the tuner measures the four block orders of
+    k_step (along the rows or down 64-wide column strips; a run of rows per XCD
+    or the hardware's order) a one-event batch runs them in turn, three steps
+    each; the plain event before it runs the first order throughout.  Same
+    arithmetic per site, so the observables agree to round-off of the
+    reductions."""
     import ipglasma_amd as I
     p = K.params("AuAu", N=192, Ny=3)
-    key = "step_waves_per_simd/N=192/events=1"
+    key = "step_block_order/N=192/events=1"
     assert key not in I.autotune_report()
     ev = I.Event(p, seed=41)
     tries = 0
