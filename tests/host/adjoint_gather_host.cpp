@@ -4,7 +4,7 @@
 #include <algorithm>
 #include <vector>
 
-#include "../../ipglasma_amd/csrc/adjoint.hpp"
+#include "adjoint_scatter.hpp"
 
 using namespace ipgad;
 

@@ -1,7 +1,7 @@
-// Host build of ipglasma_amd/csrc/adjoint.hpp: the per-site forward and
-// reverse functions over flat arrays (matrices as 18 doubles, row-major,
-// interleaved re/im), for finite-difference checks.
-#include "../../ipglasma_amd/csrc/adjoint.hpp"
+// Host build of ipglasma_amd/csrc/adjoint.hpp and of adjoint_scatter.hpp: the
+// per-site forward and reverse functions over flat arrays (matrices as 18
+// doubles, row-major, interleaved re/im), for finite-difference checks.
+#include "adjoint_scatter.hpp"
 
 using namespace ipgad;
 

@@ -1,5 +1,6 @@
 """The per-site reverse-mode functions of the leapfrog step and of T^tautau
-(ipglasma_amd/csrc/adjoint.hpp), built for the host, against central finite
+(ipglasma_amd/csrc/adjoint.hpp; the pi and E updates, which check the kernels'
+gathered sums, host/adjoint_scatter.hpp), built for the host, against central finite
 differences of their own forward functions: for random inputs x, output
 cotangent yb and direction d, Re<xb, d> = d/dh Re tr(yb^+ f(x + h d))."""
 import ctypes as C
