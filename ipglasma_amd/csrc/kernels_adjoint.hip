@@ -592,7 +592,8 @@ struct StepAcc {
 // in a role: phi and pi; U_x and E1; U_y and E2; the loops below both links
 // (handed over through LDS), ~1100-1300 FP64 multiply-adds a lane each.
 // FP64 issue and the latency of dependent products at two waves per SIMD bound
-// it (243 planes of unique traffic: 510 MB at N = 512, ~105 us as a copy).
+// it (243 planes of unique traffic: 510 MB at N = 512, ~105 us as a copy; the
+// counters read 598).
 // Measured per step, N = 192 / 256 / 512: what each site sends to its
 // neighbours written out and gathered by the next step (252 planes a set) 59 /
 // 82 / 368 us; this gather with every role loading its own matrices 39 / 53 /

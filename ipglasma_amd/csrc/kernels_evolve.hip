@@ -146,8 +146,9 @@ __device__ __forceinline__ H3 st_he(const StageRow* f, int q, const double* end,
 // One thread per site with everything in registers took 382 of them, one
 // wavefront per SIMD, whose chain of loads and products set the pace: 17 us a
 // launch at N = 128 (64 blocks of 256 sites left 192 CUs idle), 26 us at
-// N = 256, 83 us at N = 512; in roles 8.1, 20.4 and 65.6 us (302 MB of fields
-// read and written at N = 512: 4.6 TB/s, a large device copy runs at 4.9).
+// N = 256, 83 us at N = 512; in roles 7.9, 19.6 and 62.2 us (302 MB of fields
+// read and written at N = 512: 4.85 TB/s, a large device copy runs at 4.9; the
+// counters read 305 MB in order 0, the neighbour rows come from the L2).
 // Also measured: each role loading its own matrices (168 registers, three
 // waves per SIMD) 8.7, 20.7, 71 us; at 128 registers it spills (131 us);
 // only row i staged 8.0, 21.6, 68 us; blocks that stay and fetch the next
@@ -155,6 +156,9 @@ __device__ __forceinline__ H3 st_he(const StageRow* f, int q, const double* end,
 // order (the tuner's choice; the same results): bit 0: blocks follow each
 // other down 64-wide column strips (N a multiple of 64) instead of along the
 // rows; bit 1: in the hardware's block order instead of a run of rows per XCD.
+// Order 0 is the fastest or level from N = 128 to 768 (58 us at N = 512 against
+// 63, 61 and 75 in the tuner's back-to-back launches): there the others fetch
+// 31, 31 and 196 MB more, rows that another XCD's L2 holds.
 __global__ __launch_bounds__(4 * kRoleSites, 2) void k_step(const EvDesc* __restrict__ evs, int nev, int it, int b0,
                                                             int order) {
     // b0: first block of a launch that covers one event's blocks only (a
