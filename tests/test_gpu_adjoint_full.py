@@ -13,14 +13,13 @@ reference's stopping rule Sum|F| <= 1e-6): the links are then solved to
 round-off, so the forward map is smooth at the scale of the differences and
 the implicit-function gradient is exact.
 
-Error measure.  dE/deta carries round-off of about 1e-13 of its value from
-the depth of the chain (50 slices of exponentials, the root finder, 35
-steps), so a central difference carries about 1e-13 |dE/deta| / h: ~1e-4
-absolute at h = 1e-6 (dE/deta ~ 700 GeV), which exceeds 1e-6 of a
-directional derivative whenever that is below ~100.  The directional
-derivatives of random directions are ~50 on average with some near 0, so
-the error is measured against the size of the gradient along the
-directions: |adjoint - difference| <= 5e-6 rms(differences) for every
+Error measure.  dE/deta carries round-off from the depth of the chain (50
+slices of exponentials, the root finder, 35 steps), which a central difference
+divides by h = 1e-6.  The directional derivatives of random directions are ~50
+on average with some near 0, so the error is measured against the size of the
+gradient along the directions (about 1e-7 of it is seen, as much as the
+differences at h and 2h are apart; the bounds below were set for a round-off of
+1e-13 of dE/deta ~ 700 GeV): |adjoint - difference| <= 5e-6 rms(differences) for every
 direction, and the root-mean-square error <= 2e-6 rms(differences) or, when
 the differences' own round-off is larger, twice the root-mean-square
 distance between the differences at h and at 2h (the same round-off, half
